@@ -199,7 +199,7 @@ int upload(llmdot_hip_ctx* ctx, const std::string& key, uint32_t type, const voi
 // ======================================================= allocation-free ==
 // llmdot_hip_sample_noalloc keeps its scratch in this file-scope device array
 // instead of allocating: the sampler's work vector (sample_work_floats(n):
-// the probabilities and the top-p sort scratch, 9 floats per logit), the
+// 9 floats per logit and the slices' scratch), the
 // argmax candidates (one per 4096 logits) and two words (the draw counter and
 // the uniform draw).  Each device holds its own copy until the process ends;
 // its address is looked up once per device (with that device current) when a
@@ -207,13 +207,11 @@ int upload(llmdot_hip_ctx* ctx, const std::string& key, uint32_t type, const voi
 namespace {
 constexpr int NOALLOC_MAX_N = 262144;                                  // logits per call
 constexpr int NOALLOC_CAND = NOALLOC_MAX_N / 4096;                     // argmax_grid(NOALLOC_MAX_N)
-constexpr size_t NOALLOC_WORK = sizeof(float) * (((size_t)NOALLOC_MAX_N + 1) & ~(size_t)1) +
-                                sizeof(float) * 8 * (size_t)NOALLOC_MAX_N;  // sample_work_floats(NOALLOC_MAX_N)
-static_assert(NOALLOC_WORK == sizeof(float) * sample_work_floats(NOALLOC_MAX_N), "sampler work size");
+constexpr size_t NOALLOC_WORK = sizeof(float) * sample_work_floats(NOALLOC_MAX_N);
 constexpr size_t NOALLOC_CAND_VAL = NOALLOC_WORK;                      // float[NOALLOC_CAND]
 constexpr size_t NOALLOC_CAND_IDX = NOALLOC_CAND_VAL + 4 * NOALLOC_CAND;   // int32[NOALLOC_CAND]
 constexpr size_t NOALLOC_INTS = NOALLOC_CAND_IDX + 4 * NOALLOC_CAND;   // [0] draw counter, [1] draw bits
-constexpr size_t NOALLOC_BYTES = NOALLOC_INTS + 256;                   // 9 MiB + 768 B
+constexpr size_t NOALLOC_BYTES = NOALLOC_INTS + 256;
 constexpr int NOALLOC_MAX_DEVICES = 64;
 // Elements of each prefill K-part buffer: a split keeps tiles (of 128 x 128)
 // x parts <= 512 (prefill_ksplit).

@@ -179,17 +179,32 @@ struct SampleArgs {
     int hist_base;
     const int32_t* step;      // this is draw *step - 1 (the argmax pass has advanced it)
     const float* rvals;       // uniform draws: draw s uses rvals[s]
-    float* work;              // [sample_work_floats(n)] scratch: probabilities, then the top-p scratch
+    float* work;              // [sample_work_floats(n)] scratch: softmax numerators, then the other stages' scratch
     int32_t* token_out;       // the sampled token
     int32_t* token_log;       // optional: token_log[draw] = token while draw < log_cap
     int32_t log_cap;
     int32_t* hist_out;        // optional: hist_out[hist_base + draw] = token
 };
 bool sample_supported(int n, int top_k);
-// Floats of SampleArgs::work for n logits: the probabilities, then (8-byte
-// aligned) the top-p slow path's scratch: 3n 64-bit sort slots, n ids, n values.
+// Floats of SampleArgs::work for n logits: the softmax numerators, then (8-byte
+// aligned) the top-p slow path's scratch: 3n 64-bit sort slots, n ids, n values;
+// then the SampleScratch of the launches that spread over workgroups.
+constexpr int SAMPLE_BINS = 1024;     // mass histogram: bits 20 and up of a numerator in [0, 1]
+constexpr int SAMPLE_SLICES = 128;    // slices of the vocabulary
+struct SampleScratch {
+    unsigned long long mass[SAMPLE_BINS];   // numerators' sum, 2^-40 units
+    uint64_t cand[64 * 128];                // top-k: each slice's k largest
+    int32_t count[SAMPLE_BINS];
+    float smax[SAMPLE_SLICES];              // maximum of each slice
+};
 __host__ __device__ constexpr size_t sample_comp_offset(int n) { return ((size_t)n + 1) & ~(size_t)1; }
-__host__ __device__ constexpr size_t sample_work_floats(int n) { return sample_comp_offset(n) + 8 * (size_t)n; }
+__host__ __device__ constexpr size_t sample_scratch_offset(int n) { return sample_comp_offset(n) + 8 * (size_t)n; }
+__host__ __device__ constexpr size_t sample_work_floats(int n) {
+    return sample_scratch_offset(n) + sizeof(SampleScratch) / sizeof(float);
+}
+__host__ __device__ inline SampleScratch* sample_scratch(float* work, int n) {
+    return reinterpret_cast<SampleScratch*>(work + sample_scratch_offset(n));
+}
 hipError_t launch_sample(const SampleArgs& a, hipStream_t s);
 
 // ---- prefill.hip (batched prompt processing) ----

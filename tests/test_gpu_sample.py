@@ -214,3 +214,44 @@ def test_generate_sampled(hip, tiny_image, top_k, top_p):
     g, _ = eng.generate_all(prompt, GenerationOptions(max_tokens=4, sampling=opts(0.0, top_k, top_p)))
     assert len(g) == 4
     eng.dispose()
+
+
+@pytest.mark.parametrize("n,k", [(2047, 1), (2049, 127), (131072, 128), (131073, 40), (262145, 128), (524288, 7),
+                                 (524289, 40), (32000, 129), (129, 128), (20, 19)])
+def test_top_k_slices(hip, n, k):
+    """Edges of the sliced selection: whole and ragged slices of 2048, 4096 and
+    8192, the largest k and vocabulary it takes and the first beyond them (the
+    one-workgroup selection), fewer entries in a slice than k; with a repeat
+    penalty window longer than the one kept in LDS.  Exact: a token id."""
+    x = logits_for(n, n + k)
+    recent = [int(i) for i in np.random.default_rng(k).integers(0, n, 1500)] + [int(i) for i in np.argsort(-x)[:9]]
+    for o in (opts(0.8, k), opts(0.8, k, 1.0, 1.3, 1500), opts(0.8, k, 1.0, 1.3, 64)):
+        for r in R_FEW:
+            assert hip.sample(x, o, recent, r) == ref(x, o, recent, r), (o, r)
+
+
+def test_top_k_slices_equal_values(hip):
+    """Equal logits across slices: the smaller indices win (the top-k path's
+    documented order), here all n equal or the k-th value shared by many."""
+    n, k = 10000, 40
+    o = opts(1.0, k)
+    x = np.zeros(n, np.float32)
+    for r in R_ALL:   # uniform over the first k indices: the draw is ceil(r k) - 1 within rounding
+        t = hip.sample(x, o, [], r)
+        assert 0 <= t < k and abs(t - max(0.0, np.ceil(r * k) - 1)) <= 1
+    x[5000:5010] = 3.0
+    assert hip.sample(x, o, [], 0.0) == 5000
+    assert hip.sample(x, o, [], 1.0) in (k - 10 - 1, k - 10 - 2)   # the last of the zeros kept: index 29 (cum may stop short)
+
+
+@pytest.mark.parametrize("n,top_p,scale", [(8191, 0.9, 2.0), (8192, 0.9, 2.0), (8200, 0.95, 2.0), (16385, 0.5, 1.0),
+                                           (16384, 0.97, 0.05), (7, 0.9, 1.0), (9, 0.3, 1.0)])
+def test_top_p_stages(hip, n, top_p, scale):
+    """Edges of the staged softmax sum (8192 numerators a stage, tails of n mod 8)
+    and of the candidate search: a nucleus within the histogram bin's list, one
+    that needs the exact descent, one of more than 4096 tokens (all n sorted)."""
+    x = logits_for(n, n + 3, scale)
+    recent = [int(i) for i in np.argsort(-x)[:5]]
+    o = opts(0.8, 0, top_p, 1.2, 64)
+    for r in R_FEW:
+        assert hip.sample(x, o, recent, r) == ref(x, o, recent, r), r
