@@ -865,7 +865,7 @@ struct llmdot_hip_model {
     bool pf_eligible = false;
     int pf_cap = 0;
     float *pf_h = nullptr, *pf_q = nullptr, *pf_k = nullptr, *pf_v = nullptr, *pf_qr = nullptr, *pf_attn = nullptr,
-          *pf_act = nullptr, *pf_scores = nullptr, *pf_rowmax = nullptr;
+          *pf_act = nullptr, *pf_rowmax = nullptr;
     // K parts of the narrow projections (prefill_ksplit): Q, then O and down
     // (in stream order) share one buffer; K and V run at the same time as Q
     float *pf_parts_q = nullptr, *pf_parts_k = nullptr, *pf_parts_v = nullptr;
@@ -1093,17 +1093,11 @@ bool prefill_check(const llmdot_hip_model* m) {
     return true;
 }
 
-int prefill_chunk_cap(const llmdot_hip_model* m) {
+int prefill_chunk_cap() {
     int cap = 2048;
     if (const char* v = getenv("LLMDOT_HIP_PREFILL_CHUNK")) {
         const int c = atoi(v);
         if (c >= 16) cap = c;
-    }
-    // fp32 KV: score scratch [heads][cap][context] fp32 within 2 GiB (the
-    // fp16-KV attention keeps its scores in registers)
-    if (!m->d.kv_fp16) {
-        const double per_tok = 4.0 * m->d.heads * (double)m->d.context;
-        while (cap > 64 && per_tok * cap > 2147483648.0) cap /= 2;
     }
     return cap;
 }
@@ -1122,7 +1116,7 @@ int ensure_prefill_ws(llmdot_hip_model* m) {
     if (m->pf_cap) return 0;
     if (int rc = ensure_side_streams(m->ctx)) return rc;
     const auto& d = m->d;
-    const int cap = prefill_chunk_cap(m);
+    const int cap = prefill_chunk_cap();
     const size_t qdim = (size_t)d.heads * d.head_dim, kvdim = (size_t)d.kv_heads * d.head_dim;
     const size_t kmax = std::max({(size_t)d.hidden, qdim, (size_t)d.ffn});
     void* p;
@@ -1139,10 +1133,6 @@ int ensure_prefill_ws(llmdot_hip_model* m) {
     if ((rc = A(4 * PF_PARTS_MAX, &p))) return rc; m->pf_parts_q = (float*)p;
     if ((rc = A(4 * PF_PARTS_MAX, &p))) return rc; m->pf_parts_k = (float*)p;
     if ((rc = A(4 * PF_PARTS_MAX, &p))) return rc; m->pf_parts_v = (float*)p;
-    if (!d.kv_fp16) {
-        if ((rc = A(4 * (size_t)d.heads * cap * (size_t)d.context, &p))) return rc;
-        m->pf_scores = (float*)p;
-    }
     if ((rc = A(4 * (size_t)d.heads * cap, &p))) return rc; m->pf_rowmax = (float*)p;
     if ((rc = A(2 * cap * kmax, &p))) return rc; m->pf_planes.xh = (_Float16*)p;
     if ((rc = A(2 * cap * kmax, &p))) return rc; m->pf_planes.xl = (_Float16*)p;
@@ -1224,8 +1214,8 @@ int enqueue_prefill_chunk(llmdot_hip_model* m, int T, int pos0) {
         aa.kcache = m->kcache + (size_t)l * m->kv_layer_bytes;
         aa.vcache = m->vcache + (size_t)l * m->kv_layer_bytes;
         aa.cos_tab = m->cos_tab; aa.sin_tab = m->sin_tab;
-        aa.scores = m->pf_scores; aa.rowmax = m->pf_rowmax; aa.out = m->pf_attn;
-        aa.T = T; aa.pos0 = pos0; aa.ld_scores = d.context;
+        aa.rowmax = m->pf_rowmax; aa.out = m->pf_attn;
+        aa.T = T; aa.pos0 = pos0;
         aa.heads = d.heads; aa.kv_heads = d.kv_heads; aa.head_dim = d.head_dim; aa.rope_half = m->rope_half;
         aa.context = d.context; aa.kv_fp16 = d.kv_fp16;
         aa.q_norm = w.q_norm_f; aa.k_norm = w.k_norm_f; aa.eps = d.eps;

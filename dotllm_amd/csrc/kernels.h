@@ -224,15 +224,14 @@ struct PfAttnArgs {
     void* vcache;
     const float* cos_tab;     // [context][rope_half]
     const float* sin_tab;
-    float* scores;            // [heads][T][ld_scores]
-    float* rowmax;            // [heads][T]
+    float* rowmax;            // [heads][T] (64-query kernels)
     float* out;               // [T][heads*head_dim]
-    int T, pos0, ld_scores, heads, kv_heads, head_dim, rope_half, context, kv_fp16;
+    int T, pos0, heads, kv_heads, head_dim, rope_half, context, kv_fp16;
     // q, k and v as sums of q_split (k_split, v_split) K parts, q_part elements apart
     int q_split, k_split, v_split;
     int64_t q_part, k_part, v_part;
     // per-head Q/K RmsNorm weights [head_dim] applied before RoPE (null: none)
-    // with eps; SlidingWindow (0: every earlier position; fp16 KV path only)
+    // with eps; SlidingWindow (0: every earlier position)
     const float *q_norm, *k_norm;
     float eps;
     int window;
@@ -263,6 +262,8 @@ hipError_t launch_prefill_add_parts(float* h, const float* parts, int nparts, in
                                     hipStream_t s);
 hipError_t launch_prefill_rope_kv(const PfAttnArgs& a, hipStream_t s);
 hipError_t launch_prefill_attention(const PfAttnArgs& a, hipStream_t s);
+// prefill_attn.hip: the same with 16 queries per workgroup, its wavefronts over the keys.
+hipError_t launch_prefill_attn_wave(const PfAttnArgs& a, hipStream_t s);
 // Embedding rows tokens[0..T) (device ids) into out[T][hidden].
 hipError_t launch_embed_rows(const uint8_t* table, uint32_t type, int hidden, const int32_t* tokens, int T, float* out,
                              hipStream_t s);

@@ -896,163 +896,6 @@ __global__ __launch_bounds__(WG) void pf_add_parts_kernel(float* __restrict__ h,
 constexpr int AQ = 64;   // queries per workgroup
 constexpr int AK = 64;   // keys per tile
 
-template <int HD>
-__device__ __forceinline__ void load_kv_tile(float (*dst)[HD + 4], const void* cache, int64_t base, int j0, int jmax,
-                                             int fp16) {
-    // AK rows of HD elements, 4 per thread per pass
-    for (int c = threadIdx.x; c < AK * HD / 4; c += WG) {
-        const int r = c / (HD / 4), q = c - r * (HD / 4);
-        const int j = min(j0 + r, jmax);
-        const int64_t idx = base + (int64_t)j * HD + 4 * q;
-        float4 v;
-        if (fp16) {
-            const uint2 u = *reinterpret_cast<const uint2*>(reinterpret_cast<const _Float16*>(cache) + idx);
-            v.x = (float)__builtin_bit_cast(_Float16, (uint16_t)(u.x & 0xFFFFu));
-            v.y = (float)__builtin_bit_cast(_Float16, (uint16_t)(u.x >> 16));
-            v.z = (float)__builtin_bit_cast(_Float16, (uint16_t)(u.y & 0xFFFFu));
-            v.w = (float)__builtin_bit_cast(_Float16, (uint16_t)(u.y >> 16));
-        } else {
-            v = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(cache) + idx);
-        }
-        *reinterpret_cast<float4*>(&dst[r][4 * q]) = v;
-    }
-}
-
-// Scores (q . K_j) / sqrt(hd) of 64 queries of one q head against every key
-// j <= pos0 + t, into the score scratch, and each query's maximum.
-template <int HD>
-__global__ __launch_bounds__(WG) void pf_attn_scores_kernel(PfAttnArgs a) {
-    __shared__ __attribute__((aligned(16))) float Qs[AQ][HD + 4];
-    __shared__ __attribute__((aligned(16))) float Ks[AK][HD + 4];
-    const int t0 = blockIdx.x * AQ, h = blockIdx.y, kvh = h / (a.heads / a.kv_heads);
-    const int qdim = a.heads * HD;
-    const int tid = threadIdx.x, tq = tid >> 4, tk = tid & 15;
-    for (int c = tid; c < AQ * HD / 4; c += WG) {
-        const int r = c / (HD / 4), q = c - r * (HD / 4);
-        const int t = min(t0 + r, a.T - 1);
-        *reinterpret_cast<float4*>(&Qs[r][4 * q]) =
-            *reinterpret_cast<const float4*>(a.qr + (int64_t)t * qdim + h * HD + 4 * q);
-    }
-    const int nkeys = a.pos0 + min(t0 + AQ, a.T);   // keys 0 .. pos0 + last query
-    const int64_t kbase = (int64_t)kvh * a.context * HD;
-    const float inv_sqrt = 1.0f / sqrtf((float)HD);
-    float rmax[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    for (int j0 = 0; j0 < nkeys; j0 += AK) {
-        __syncthreads();
-        load_kv_tile<HD>(Ks, a.kcache, kbase, j0, nkeys - 1, a.kv_fp16);
-        __syncthreads();
-        float s[4][4];
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) s[i][j] = 0.f;
-#pragma unroll 4
-        for (int d = 0; d < HD; d += 4) {
-            float4 qv[4], kv[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) qv[i] = *reinterpret_cast<const float4*>(&Qs[4 * tq + i][d]);
-#pragma unroll
-            for (int j = 0; j < 4; j++) kv[j] = *reinterpret_cast<const float4*>(&Ks[4 * tk + j][d]);
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-                    s[i][j] += qv[i].x * kv[j].x + qv[i].y * kv[j].y + qv[i].z * kv[j].z + qv[i].w * kv[j].w;
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int t = t0 + 4 * tq + i;
-            if (t >= a.T) continue;
-            const int p = a.pos0 + t;
-            float* srow = a.scores + ((int64_t)h * a.T + t) * a.ld_scores;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int key = j0 + 4 * tk + j;
-                if (key <= p) {
-                    const float sc = s[i][j] * inv_sqrt;
-                    srow[key] = sc;
-                    rmax[i] = fmaxf(rmax[i], sc);
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        float m = rmax[i];
-        m = max16(m);
-        const int t = t0 + 4 * tq + i;
-        if (tk == 0 && t < a.T) a.rowmax[(int64_t)h * a.T + t] = m;
-    }
-}
-
-// Softmax (VectorMath.Softmax, VM:215-258: ExpApprox(s - max) on the first
-// 8 floor(n/8) scores, expf on the tail) and out = sum_j e_j V_j / sum_j e_j
-// for 64 queries of one q head.
-template <int HD>
-__global__ __launch_bounds__(WG) void pf_attn_pv_kernel(PfAttnArgs a) {
-    constexpr int DPT = HD / 16;
-    __shared__ __attribute__((aligned(16))) float Vs[AK][HD + 4];
-    __shared__ float Es[AQ][AK + 1];
-    __shared__ float Ms[AQ];
-    const int t0 = blockIdx.x * AQ, h = blockIdx.y, kvh = h / (a.heads / a.kv_heads);
-    const int qdim = a.heads * HD;
-    const int tid = threadIdx.x, tq = tid >> 4, td = tid & 15;
-    if (tid < AQ) Ms[tid] = a.rowmax[(int64_t)h * a.T + min(t0 + tid, a.T - 1)];
-    const int nkeys = a.pos0 + min(t0 + AQ, a.T);
-    const int64_t vbase = (int64_t)kvh * a.context * HD;
-    float acc[4][DPT], z[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int d = 0; d < DPT; d++) acc[i][d] = 0.f;
-    for (int j0 = 0; j0 < nkeys; j0 += AK) {
-        __syncthreads();
-        load_kv_tile<HD>(Vs, a.vcache, vbase, j0, nkeys - 1, a.kv_fp16);
-        for (int c = tid; c < AQ * AK; c += WG) {
-            const int qi = c >> 6, kj = c & 63;
-            const int t = t0 + qi, key = j0 + kj;
-            float e = 0.f;
-            if (t < a.T) {
-                const int n = a.pos0 + t + 1, n8 = n & ~7;
-                if (key < n) {
-#pragma clang fp contract(off)
-                    const float x = a.scores[((int64_t)h * a.T + t) * a.ld_scores + key] - Ms[qi];
-                    e = key < n8 ? exp_approx(x) : expf(x);
-                }
-            }
-            Es[qi][kj] = e;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int k = 0; k < 4; k++) z[i] += Es[4 * tq + i][4 * td + k];
-#pragma unroll 4
-        for (int kj = 0; kj < AK; kj++) {
-            float ev[4], vv[DPT];
-#pragma unroll
-            for (int i = 0; i < 4; i++) ev[i] = Es[4 * tq + i][kj];
-#pragma unroll
-            for (int d = 0; d < DPT; d++) vv[d] = Vs[kj][td * DPT + d];
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int d = 0; d < DPT; d++) acc[i][d] += ev[i] * vv[d];
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        float zz = z[i];
-        zz = sum16(zz);
-        const int t = t0 + 4 * tq + i;
-        if (t < a.T) {
-            const float inv = 1.0f / zz;
-#pragma unroll
-            for (int d = 0; d < DPT; d++) a.out[(int64_t)t * qdim + h * HD + td * DPT + d] = acc[i][d] * inv;
-        }
-    }
-}
-
 // ---- attention on MFMA (fp16 KV cache) ----
 //
 // K and V are fp16 in the cache, so they are exact MFMA operands; q (per
@@ -1343,12 +1186,10 @@ hipError_t launch_gemm_fmt(int epi, PfGemmArgs a, hipStream_t s) {
 template <int HD>
 hipError_t launch_attn_hd(const PfAttnArgs& a, hipStream_t s) {
     const dim3 grid((a.T + AQ - 1) / AQ, a.heads);
-    if (a.kv_fp16) pf_attn_max_mfma<HD><<<grid, WG, 0, s>>>(a);
-    else pf_attn_scores_kernel<HD><<<grid, WG, 0, s>>>(a);
+    pf_attn_max_mfma<HD><<<grid, WG, 0, s>>>(a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if (a.kv_fp16) pf_attn_pv_mfma<HD><<<grid, WG, 0, s>>>(a);
-    else pf_attn_pv_kernel<HD><<<grid, WG, 0, s>>>(a);
+    pf_attn_pv_mfma<HD><<<grid, WG, 0, s>>>(a);
     return hipGetLastError();
 }
 
@@ -1444,6 +1285,16 @@ int prefill_ksplit(uint32_t type, int M, int N, int K) {
 
 hipError_t launch_prefill_attention(const PfAttnArgs& a, hipStream_t s) {
     if (a.T <= 0 || a.heads % a.kv_heads) return hipErrorInvalidValue;
+    // fp16 cache: the 64-query kernels read each K / V tile once per 64 queries
+    // and win where their workgroups fill the chip twice (us per layer, both
+    // passes against the wave kernel: 512 workgroups 88 / 107 (1024 tokens, 32
+    // heads of 128), 76 / 73 (of 96), 1024 workgroups 197 / 343), or once with
+    // long key loops (256 workgroups of 4012 keys: 289 / 311).  Below that
+    // their workgroups walk the keys alone (23 tokens behind 1800: 136 / 40;
+    // 128 behind 3900: 276 / 88; 256 workgroups of 512 keys 35 / 19, of 2048
+    // keys 119 / 58; 416 of 777: 60 / 36).
+    const int wgs = (a.T + AQ - 1) / AQ * a.heads;
+    if (!a.kv_fp16 || wgs < 256 || (wgs < 512 && a.pos0 + a.T <= 2048)) return launch_prefill_attn_wave(a, s);
     switch (a.head_dim) {
     case 64: return launch_attn_hd<64>(a, s);
     case 96: return launch_attn_hd<96>(a, s);

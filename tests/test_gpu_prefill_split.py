@@ -25,3 +25,20 @@ def test_prefill_partial_rotation(hip, monkeypatch, rot):
     monkeypatch.setattr(synth, "metadata", metadata)
     img = synth.build_image("tiny", seed=1234, context=96)
     _prompt_check(hip, img, synth.prompt(32000, 40, seed=5), 96, True, [0, 3])
+
+
+@pytest.mark.parametrize("n,split,kv_fp16", [(2, None, False), (17, None, True), (33, None, False), (49, 47, True),
+                                             (300, 283, False), (300, 283, True)])
+def test_prefill_attention_key_split(hip, oracle_threads, n, split, kv_fp16):  # noqa: F811
+    """Heads of 96 (two layers of the Phi-3-mini shape): fewer keys than the
+    wavefronts' steps, a last query block of one row, a chunk behind a cache."""
+    spec = dict(synth.SPECS["phi3mini"], layers=2)
+    img = synth.build_image("phi3mini", seed=1234, spec=spec, context=320)
+    _prompt_check(hip, img, synth.prompt(32064, n, seed=7), 320, kv_fp16, [0, 1], split=split)
+
+
+def test_prefill_attention_512_queries_groups(hip, oracle_threads):  # noqa: F811
+    """Four wavefronts a workgroup, query groups of 2, heads of 128."""
+    spec = dict(synth.SPECS["small5"], layers=1)
+    img = synth.build_image("small5", seed=1234, spec=spec, context=600)
+    _prompt_check(hip, img, synth.prompt(32000, 530, seed=7), 600, False, [0])
