@@ -94,7 +94,7 @@ struct llmdot_hip_ctx {
     hipStream_t stream = nullptr;
     std::unordered_map<std::string, Weight> weights;
     DevBuf scratch[6];
-    DevBuf planes[5];            // batched MatMul: activation planes (xh, xl, sh, sl, xinv)
+    DevBuf planes[6];            // batched MatMul: activation planes (xh, xl, sh, sl, xinv)
     int32_t* am_ints = nullptr;  // [0] token_out
     float* am_val = nullptr;
     int32_t* am_idx = nullptr;
@@ -213,8 +213,7 @@ constexpr size_t NOALLOC_CAND_IDX = NOALLOC_CAND_VAL + 4 * NOALLOC_CAND;   // in
 constexpr size_t NOALLOC_INTS = NOALLOC_CAND_IDX + 4 * NOALLOC_CAND;   // [0] draw counter, [1] draw bits
 constexpr size_t NOALLOC_BYTES = NOALLOC_INTS + 256;
 constexpr int NOALLOC_MAX_DEVICES = 64;
-// Elements of each prefill K-part buffer: a split keeps tiles (of 128 x 128)
-// x parts <= 512 (prefill_ksplit).
+// Elements of each prefill K-part buffer (prefill_plan keeps to it).
 constexpr int64_t PF_PARTS_MAX = 512LL * 128 * 128;
 
 __attribute__((used)) __device__ __align__(256) uint8_t scratch[NOALLOC_BYTES];
@@ -438,7 +437,17 @@ int matmul_common(llmdot_hip_ctx* ctx, const float* a, const void* b, float* res
         PfPlanes pl;
         if (int rc = ctx_planes(ctx, (int)a_rows, a_cols, &pl)) return rc;
         HIPCHK(launch_prefill_planes(da, (int)a_rows, a_cols, nullptr, 0.f, pl, ctx->stream));
-        HIPCHK(launch_prefill_gemm(type, 0, pl, w->dev, nullptr, (int)a_rows, b_cols, a_cols, dy, b_cols, ctx->stream));
+        const int M = (int)a_rows;
+        const PfPlan plan = prefill_plan(type, M, b_cols, a_cols, PF_PARTS_MAX);
+        PfMat mat{w->dev, b_cols, dy, b_cols, 0};
+        if (plan.ksplit > 1) {
+            mat.part_stride = (result_len + 3) & ~int64_t(3);
+            HIPCHK(ctx->planes[5].ensure(sizeof(float) * (size_t)(plan.ksplit * mat.part_stride)));
+            mat.out = (float*)ctx->planes[5].p;
+        }
+        HIPCHK(launch_prefill_gemm(type, 0, pl, mat, PfMat{}, M, a_cols, plan, ctx->stream));
+        if (plan.ksplit > 1)
+            HIPCHK(launch_prefill_sum_parts(dy, false, mat.out, plan.ksplit, mat.part_stride, result_len, ctx->stream));
         return copy_out(ctx, result, dy, sizeof(float) * (size_t)result_len);
     }
     for (int64_t r = 0; r < a_rows; r++)
@@ -866,7 +875,7 @@ struct llmdot_hip_model {
     int pf_cap = 0;
     float *pf_h = nullptr, *pf_q = nullptr, *pf_k = nullptr, *pf_v = nullptr, *pf_qr = nullptr, *pf_attn = nullptr,
           *pf_act = nullptr, *pf_rowmax = nullptr;
-    // K parts of the narrow projections (prefill_ksplit): Q, then O and down
+    // K parts (prefill_plan): Q, gate, then O and down
     // (in stream order) share one buffer; K and V run at the same time as Q
     float *pf_parts_q = nullptr, *pf_parts_k = nullptr, *pf_parts_v = nullptr;
     PfPlanes pf_planes{};
@@ -1129,7 +1138,6 @@ int ensure_prefill_ws(llmdot_hip_model* m) {
     if ((rc = A(4 * cap * qdim, &p))) return rc; m->pf_qr = (float*)p;
     if ((rc = A(4 * cap * qdim, &p))) return rc; m->pf_attn = (float*)p;
     if ((rc = A(4 * cap * (size_t)d.ffn, &p))) return rc; m->pf_act = (float*)p;
-    // a K split keeps tiles x parts <= 512, so parts x rows x cols <= 512 x 128 x 128
     if ((rc = A(4 * PF_PARTS_MAX, &p))) return rc; m->pf_parts_q = (float*)p;
     if ((rc = A(4 * PF_PARTS_MAX, &p))) return rc; m->pf_parts_k = (float*)p;
     if ((rc = A(4 * PF_PARTS_MAX, &p))) return rc; m->pf_parts_v = (float*)p;
@@ -1152,64 +1160,68 @@ int enqueue_prefill_chunk(llmdot_hip_model* m, int T, int pos0) {
     hipStream_t s = m->ctx->stream;
     const int qdim = d.heads * d.head_dim, kvdim = d.kv_heads * d.head_dim;
     const PfPlanes& pl = m->pf_planes;
+    // Tile and K parts of a projection of N rows over K columns (K parts go
+    // to a buffer of PF_PARTS_MAX floats and are summed by the next kernel)
     const bool split_ok = !env_flag("LLMDOT_HIP_PF_NO_SPLIT");
-    // A STORE projection [T x N] over K columns, in K parts into `parts` when
-    // the launch has few tiles; returns the part count (1: written to out).
-    auto proj = [&](const Weight* w, int N, int K, float* out, float* parts, hipStream_t st, int* nparts) {
-        int sp = split_ok ? prefill_ksplit(w->type, T, N, K) : 1;
-        if ((int64_t)sp * T * N > PF_PARTS_MAX) sp = 1;
-        *nparts = sp;
-        if (sp == 1) return launch_prefill_gemm(w->type, 0, pl, w->dev, nullptr, T, N, K, out, N, st);
-        return launch_prefill_gemm(w->type, 0, pl, w->dev, nullptr, T, N, K, parts, N, st, sp, (int64_t)T * N);
+    auto plan_of = [&](const Weight* w, int N, int K) {
+        return prefill_plan(w->type, T, N, K, split_ok ? PF_PARTS_MAX : 0);
     };
-    // h += the [T x hidden] projection: in place, or its K parts then their sum
+    // one matrix: [T x rows] into out, or its parts
+    auto mat = [&](const Weight* w, int rows, float* out, float* parts, const PfPlan& p) {
+        return PfMat{w->dev, rows, p.ksplit > 1 ? parts : out, rows, (int64_t)T * rows};
+    };
+    // h += the [T x hidden] projection: in place, or left as `pending` parts
+    // for the next norm's planes to add
+    int pending = 0;
+    const int64_t hstride = (int64_t)T * d.hidden;
     auto proj_add = [&](const Weight* w, int K) {
-        int sp = split_ok ? prefill_ksplit(w->type, T, d.hidden, K) : 1;
-        if ((int64_t)sp * T * d.hidden > PF_PARTS_MAX) sp = 1;
-        if (sp == 1) return launch_prefill_gemm(w->type, 1, pl, w->dev, nullptr, T, d.hidden, K, m->pf_h, d.hidden, s);
-        const int64_t n = (int64_t)T * d.hidden;
-        hipError_t e = launch_prefill_gemm(w->type, 0, pl, w->dev, nullptr, T, d.hidden, K, m->pf_parts_q, d.hidden, s,
-                                           sp, n);
-        return e != hipSuccess ? e : launch_prefill_add_parts(m->pf_h, m->pf_parts_q, sp, n, n, s);
+        const PfPlan p = plan_of(w, d.hidden, K);
+        if (p.ksplit == 1 && p.tm != 32)
+            return launch_prefill_gemm(w->type, 1, pl, PfMat{w->dev, d.hidden, m->pf_h, d.hidden, 0}, PfMat{}, T, K, p, s);
+        pending = p.ksplit;
+        return launch_prefill_gemm(w->type, 0, pl, PfMat{w->dev, d.hidden, m->pf_parts_q, d.hidden, hstride}, PfMat{}, T, K,
+                                   p, s);
     };
-    // Q and K (same type) as one launch where neither would be split in K:
-    // their row tiles then share the CUs in one grid instead of K's narrow
-    // launch running beside Q's (LLMDOT_HIP_PF_QK_PAIR=0 turns this off)
-    const bool pair_ok = !env_is_zero("LLMDOT_HIP_PF_QK_PAIR") && qdim % 128 == 0;
-    auto qk_pair = [&](const LayerW& w) {
-        return pair_ok && w.q->type == w.k->type && prefill_ksplit(w.q->type, T, qdim, d.hidden) == 1 &&
-               prefill_ksplit(w.k->type, T, kvdim, d.hidden) == 1;
+    auto norm_planes = [&](const float* norm_w) {
+        const int n = pending;
+        pending = 0;
+        if (n) return launch_prefill_planes_add(m->pf_h, m->pf_parts_q, n, hstride, T, d.hidden, norm_w, d.eps, pl, s);
+        return launch_prefill_planes(m->pf_h, T, d.hidden, norm_w, d.eps, pl, s);
     };
+    // Q and K (same type) as one launch: their row tiles then share the CUs in
+    // one grid instead of K's narrow launch running beside Q's
+    // (LLMDOT_HIP_PF_QK_PAIR=0 turns this off)
+    const bool pair_ok = !env_is_zero("LLMDOT_HIP_PF_QK_PAIR");
     HIPCHK(launch_embed_rows(m->embd->dev, m->embd->type, d.hidden, m->pf_tokens, T, m->pf_h, s));
     for (int l = 0; l < d.layers; l++) {
         const LayerW& w = m->L[l];
-        HIPCHK(launch_prefill_planes(m->pf_h, T, d.hidden, w.attn_norm_f, d.eps, pl, s));
+        HIPCHK(norm_planes(w.attn_norm_f));
         // Q, K and V read the same planes and write separate buffers: V runs
-        // on a side stream beside Q and K (one launch where qk_pair allows,
-        // else K on the other side stream; K and V alone fill half the CUs)
+        // on a side stream beside Q and K (one launch where they have one
+        // type, else K on the other side stream)
         llmdot_hip_ctx* c = m->ctx;
-        int nq = 1, nk = 1, nv = 1;
+        const bool same = w.q->type == w.k->type && qdim % 128 == 0, pair = same && pair_ok;
+        const PfPlan pv = plan_of(w.v, kvdim, d.hidden);
+        const PfPlan pq = plan_of(w.q, same ? qdim + kvdim : qdim, d.hidden);
+        const PfPlan pk = same ? pq : plan_of(w.k, kvdim, d.hidden);
+        const PfMat mq = mat(w.q, qdim, m->pf_q, m->pf_parts_q, pq), mk = mat(w.k, kvdim, m->pf_k, m->pf_parts_k, pk),
+                    mv = mat(w.v, kvdim, m->pf_v, m->pf_parts_v, pv);
         HIPCHK(hipEventRecord(c->fork, s));
         HIPCHK(hipStreamWaitEvent(c->side[1], c->fork, 0));
-        HIPCHK(proj(w.v, kvdim, d.hidden, m->pf_v, m->pf_parts_v, c->side[1], &nv));
+        HIPCHK(launch_prefill_gemm(w.v->type, 0, pl, mv, PfMat{}, T, d.hidden, pv, c->side[1]));
         HIPCHK(hipEventRecord(c->join[1], c->side[1]));
-        if (qk_pair(w)) {   // Q and K in one launch, of 128-token tiles
-            HIPCHK(launch_prefill_gemm_pair(w.q->type, pl, w.q->dev, qdim, m->pf_q, qdim, w.k->dev, kvdim, m->pf_k,
-                                            kvdim, T, d.hidden, s));
-        } else {
+        if (!pair) {
             HIPCHK(hipStreamWaitEvent(c->side[0], c->fork, 0));
-            HIPCHK(proj(w.k, kvdim, d.hidden, m->pf_k, m->pf_parts_k, c->side[0], &nk));
+            HIPCHK(launch_prefill_gemm(w.k->type, 0, pl, mk, PfMat{}, T, d.hidden, pk, c->side[0]));
             HIPCHK(hipEventRecord(c->join[0], c->side[0]));
-            HIPCHK(proj(w.q, qdim, d.hidden, m->pf_q, m->pf_parts_q, s, &nq));
-            HIPCHK(hipStreamWaitEvent(s, c->join[0], 0));
         }
+        HIPCHK(launch_prefill_gemm(w.q->type, 0, pl, mq, pair ? mk : PfMat{}, T, d.hidden, pq, s));
+        if (!pair) HIPCHK(hipStreamWaitEvent(s, c->join[0], 0));
         HIPCHK(hipStreamWaitEvent(s, c->join[1], 0));
         PfAttnArgs aa{};
-        aa.q = nq > 1 ? m->pf_parts_q : m->pf_q;
-        aa.k = nk > 1 ? m->pf_parts_k : m->pf_k;
-        aa.v = nv > 1 ? m->pf_parts_v : m->pf_v;
-        aa.q_split = nq; aa.k_split = nk; aa.v_split = nv;
-        aa.q_part = (int64_t)T * qdim; aa.k_part = (int64_t)T * kvdim; aa.v_part = (int64_t)T * kvdim;
+        aa.q = mq.out; aa.k = mk.out; aa.v = mv.out;
+        aa.q_split = pq.ksplit; aa.k_split = pk.ksplit; aa.v_split = pv.ksplit;
+        aa.q_part = mq.part_stride; aa.k_part = mk.part_stride; aa.v_part = mv.part_stride;
         aa.qr = m->pf_qr;
         aa.kcache = m->kcache + (size_t)l * m->kv_layer_bytes;
         aa.vcache = m->vcache + (size_t)l * m->kv_layer_bytes;
@@ -1224,10 +1236,27 @@ int enqueue_prefill_chunk(llmdot_hip_model* m, int T, int pos0) {
         HIPCHK(launch_prefill_attention(aa, s));
         HIPCHK(launch_prefill_planes(m->pf_attn, T, qdim, nullptr, 0.f, pl, s));
         HIPCHK(proj_add(w.o, qdim));
-        HIPCHK(launch_prefill_planes(m->pf_h, T, d.hidden, w.ffn_norm_f, d.eps, pl, s));
-        HIPCHK(launch_prefill_gemm(w.gate->type, 2, pl, w.gate->dev, w.up->dev, T, d.ffn, d.hidden, m->pf_act, d.ffn, s));
-        HIPCHK(launch_prefill_planes(m->pf_act, T, d.ffn, nullptr, 0.f, pl, s));
+        HIPCHK(norm_planes(w.ffn_norm_f));
+        PfPlan pg{128, 1};   // one launch of gate and up tiles
+        if (w.gate->type == w.up->type && d.ffn % 128 == 0 && split_ok)
+            pg = prefill_swiglu_plan(w.gate->type, T, d.ffn, d.hidden, PF_PARTS_MAX);
+        if (pg.ksplit > 1 || pg.tm != 128) {
+            // gate and up as K parts, joined by the planes
+            const int64_t st = (int64_t)T * d.ffn;
+            const PfMat mg{w.gate->dev, d.ffn, m->pf_parts_q, d.ffn, st}, mu{w.up->dev, d.ffn, m->pf_parts_k, d.ffn, st};
+            HIPCHK(launch_prefill_gemm(w.gate->type, 0, pl, mg, mu, T, d.hidden, pg, s));
+            HIPCHK(launch_prefill_planes_swiglu(mg.out, mu.out, pg.ksplit, st, T, d.ffn, pl, s));
+        } else {
+            HIPCHK(launch_prefill_gemm(w.gate->type, 2, pl, PfMat{w.gate->dev, d.ffn, m->pf_act, d.ffn, 0},
+                                       PfMat{w.up->dev, d.ffn, nullptr, d.ffn, 0}, T, d.hidden, pg, s));
+            HIPCHK(launch_prefill_planes(m->pf_act, T, d.ffn, nullptr, 0.f, pl, s));
+        }
         HIPCHK(proj_add(w.down, d.ffn));
+    }
+    // the head reads the last token's row only
+    if (pending) {
+        const size_t o = (size_t)(T - 1) * d.hidden;
+        HIPCHK(launch_prefill_sum_parts(m->pf_h + o, true, m->pf_parts_q + o, pending, hstride, d.hidden, s));
     }
     return 0;
 }

@@ -237,28 +237,44 @@ struct PfAttnArgs {
     int window;
 };
 bool prefill_gemm_supported(uint32_t type, int cols);
-// Optional RmsNorm (norm_w non-null) of each row of x, then its planes.
+// Optional RmsNorm (norm_w non-null) of each row of x (K <= 16384), then its planes.
 hipError_t launch_prefill_planes(const float* x, int M, int K, const float* norm_w, float eps, const PfPlanes& p,
                                  hipStream_t s);
-// out[M][ldo] (=, += for epi 1, SiLU(gate) * up for epi 2 with w = gate, w2 = up)
-// of the planes times the [N][K] weight blocks, transposed.  ksplit > 1 (STORE
-// only): K in ksplit parts of whole blocks, part p written at out + p * part_stride.
-hipError_t launch_prefill_gemm(uint32_t type, int epi, const PfPlanes& p, const uint8_t* w, const uint8_t* w2, int M,
-                               int N, int K, float* out, int ldo, hipStream_t s, int ksplit = 1,
-                               int64_t part_stride = 0);
-// K parts for an [M x N x K] prefill GEMM: more than 1 only for launches of
-// fewer than 128 tiles, so that tiles x parts stays within 512 workgroups.
-// (Splitting the 128-tile K/V projections of a 7B-shape 2048-token prompt too
-// moved a deep-layer fp16 KV row one ulp past twice the oracle's reorder
-// floor.)
-int prefill_ksplit(uint32_t type, int M, int N, int K);
-// Two STORE products over the same planes in one launch: out[M][ldo] of the
-// [N][K] blocks w (N a multiple of 128 rows) and outb[M][ldob] of the [nb][K]
-// blocks wb, same type; each output equals launch_prefill_gemm's.
-hipError_t launch_prefill_gemm_pair(uint32_t type, const PfPlanes& p, const uint8_t* w, int N, float* out, int ldo,
-                                    const uint8_t* wb, int nb, float* outb, int ldob, int M, int K, hipStream_t s);
-// h[i] += sum over the nparts parts (stride elements apart) of parts[p][i], i < n.
-hipError_t launch_prefill_add_parts(float* h, const float* parts, int nparts, int64_t stride, int64_t n,
+// The same of h += sum of a projection's K parts [M][K] (then RmsNorm), and of
+// SiLU(gate) * up of two projections' K parts; parts stride elements apart.
+hipError_t launch_prefill_planes_add(float* h, const float* parts, int nparts, int64_t stride, int M, int K,
+                                     const float* norm_w, float eps, const PfPlanes& p, hipStream_t s);
+hipError_t launch_prefill_planes_swiglu(const float* gate, const float* up, int nparts, int64_t stride, int M, int K,
+                                        const PfPlanes& p, hipStream_t s);
+// One weight matrix of a prefill GEMM: [rows][K] blocks, its output [M][ld]
+// (K part p at out + p * part_stride).
+struct PfMat {
+    const uint8_t* w;
+    int rows;
+    float* out;
+    int ld;
+    int64_t part_stride;
+};
+// Tokens per tile (128, 64 or 32) and K parts of a prefill GEMM.
+struct PfPlan {
+    int tm, ksplit;
+};
+// The planes times wa's blocks, transposed: epi 0 stores, 1 adds to out, 2
+// stores SiLU(gate) * up with wa = gate, wb = up (out in wa).  epi 0 takes a
+// second matrix of the same type in the same launch where wa.rows is a
+// multiple of 128 (wb.w non-null); each output is the same as alone.  K parts
+// (epi 0 only) are whole blocks.
+hipError_t launch_prefill_gemm(uint32_t type, int epi, const PfPlanes& p, const PfMat& wa, const PfMat& wb, int M,
+                               int K, const PfPlan& plan, hipStream_t s);
+// Tile and K parts for an epi 0 launch of N weight rows (of both matrices)
+// and at most max_parts floats of parts.
+PfPlan prefill_plan(uint32_t type, int M, int N, int K, int64_t max_parts);
+// The same for gate and up (N rows each): {128, 1} is the epi 2 launch,
+// anything else one epi 0 launch of both into parts of at most max_parts
+// floats each.
+PfPlan prefill_swiglu_plan(uint32_t type, int M, int N, int K, int64_t max_parts);
+// out[i] = (or +=) the sum of the nparts parts (stride elements apart), i < n.
+hipError_t launch_prefill_sum_parts(float* out, bool add, const float* parts, int nparts, int64_t stride, int64_t n,
                                     hipStream_t s);
 hipError_t launch_prefill_rope_kv(const PfAttnArgs& a, hipStream_t s);
 hipError_t launch_prefill_attention(const PfAttnArgs& a, hipStream_t s);

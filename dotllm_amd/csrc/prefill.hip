@@ -33,9 +33,8 @@
 // K).  Each step's activation planes and raw weight blocks are copied
 // global -> LDS by the waves (global_load_lds, no registers) one step ahead
 // into two LDS stages; each wave then builds its weight fragments from the
-// raw bytes in LDS.  Launches that would have few tiles use 64-token tiles
-// (128 to 255 tiles) or split K into parts summed by the next kernel (under
-// 128 tiles).
+// raw bytes in LDS.  Launches with few tiles use 64- or 32-token tiles or
+// split K into parts summed by the next kernel (prefill_plan).
 #include "common.h"
 #include "kernels.h"
 
@@ -59,69 +58,157 @@ constexpr int WG = 256;
 
 // ---------------------------------------------------------------- planes --
 
-// One workgroup per token row: optional RmsNorm (VectorMath.RmsNorm, VM:308-340:
-// ss = sum x^2, inv = 1/sqrt(ss/n + eps), y = (w x) inv on the vector lanes,
-// w (x inv) on the tail), then the power-of-two scale, the two fp16 planes of
-// y s, the group sums of y (scaled by s/32) as two planes, and 1/s.
-template <bool NORM>
-__global__ __launch_bounds__(WG) void pf_planes_kernel(const float* __restrict__ x, int K, const float* __restrict__ w,
-                                                       float eps, _Float16* __restrict__ xh, _Float16* __restrict__ xl,
-                                                       _Float16* __restrict__ sh, _Float16* __restrict__ sl,
-                                                       float* __restrict__ xinv) {
-    __shared__ float red[WG / 64];
-    const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const float* row = x + (int64_t)t * K;
-    float inv = 1.f;
-    if (NORM) {
-        float ss = 0.f;
-        for (int i = tid; i < K; i += WG) {
-            const float v = row[i];
-            ss += v * v;
-        }
-        ss = wave_sum(ss);
-        if (lane == 0) red[wave] = ss;
-        __syncthreads();
-        float tot = 0.f;
+template <int V>
+struct FVec {
+    float v[V];
+    __device__ __forceinline__ void load(const float* p) {
+        if constexpr (V == 4) {
+            const f4 x = *reinterpret_cast<const f4*>(p);
 #pragma unroll
-        for (int i = 0; i < WG / 64; i++) tot += red[i];
-        __syncthreads();
-        {
-#pragma clang fp contract(off)
-            inv = 1.0f / sqrtf((tot / (float)K) + eps);
+            for (int i = 0; i < 4; i++) v[i] = x[i];
+        } else {
+            v[0] = p[0];
         }
     }
+    // parts in order, four of them in flight
+    __device__ __forceinline__ void load_parts(const float* x, int n, int64_t stride) {
+        load(x);
+        int p = 1;
+        for (; p + 3 < n; p += 4) {
+            FVec t[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) t[j].load(x + (p + j) * stride);
+#pragma unroll
+            for (int j = 0; j < 4; j++) add(t[j]);
+        }
+        for (; p < n; p++) {
+            FVec t;
+            t.load(x + p * stride);
+            add(t);
+        }
+    }
+    __device__ __forceinline__ void add(const FVec& o) {
+#pragma unroll
+        for (int i = 0; i < V; i++) v[i] += o.v[i];
+    }
+    __device__ __forceinline__ void store(float* p) const {
+        if constexpr (V == 4) *reinterpret_cast<f4*>(p) = f4{v[0], v[1], v[2], v[3]};
+        else p[0] = v[0];
+    }
+    __device__ __forceinline__ void store_kv(void* cache, int64_t idx, int fp16) const {
+        if constexpr (V == 4) {
+            if (fp16) {
+                *reinterpret_cast<h4*>(reinterpret_cast<_Float16*>(cache) + idx) =
+                    h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+            } else {
+                store(reinterpret_cast<float*>(cache) + idx);
+            }
+        } else {
+            llmdot::store_kv(cache, idx, v[0], fp16);
+        }
+    }
+};
+
+// What a row's planes are made of: the row itself, the row plus the K parts of
+// a projection (the residual add; written back), or SiLU(gate) * up of two
+// projections' K parts.
+enum PfSrc : int { SRC_ROW = 0, SRC_ADD = 1, SRC_SWIGLU = 2 };
+
+struct PfPlanesArgs {
+    float* x;              // SRC_ROW, SRC_ADD: [M][K]
+    const float *pa, *pb;  // SRC_ADD: parts; SRC_SWIGLU: gate and up parts
+    int nparts;
+    int64_t stride;
+    int K;
+    const float* w;        // RmsNorm weights (null: none)
+    float eps;
+    PfPlanes p;
+};
+
+// One workgroup of T threads per token row: optional RmsNorm (VectorMath.RmsNorm,
+// VM:308-340: ss = sum x^2, inv = 1/sqrt(ss/n + eps), y = (w x) inv on the
+// vector lanes, w (x inv) on the tail), then the power-of-two scale, the two
+// fp16 planes of y s, the group sums of y (scaled by s/32) as two planes, and
+// 1/s.  A thread holds 4 consecutive elements of each of NB blocks of 4 T in
+// registers, so the row is read once.  Bound by memory for long chunks (2048 x
+// 4096 with the norm 33 -> 13 us against reading the row again for each pass);
+// with few rows by the loads' and the two reductions' latency, hence 1024
+// threads a row up to 256 rows (23 x 4096 with the norm 11 -> 4 us; 512 rows:
+// the same with either).
+template <bool NORM, int SRC, int NB, int T>
+__global__ __launch_bounds__(T) void pf_planes_kernel(PfPlanesArgs a) {
+    __shared__ float red[2][T / 64];
+    const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, K = a.K;
     const int n8 = K & ~7;
-    auto yval = [&](int i) -> float {
-#pragma clang fp contract(off)
-        const float v = row[i];
-        if (!NORM) return v;
-        return i < n8 ? ((w[i] * v) * inv) : (w[i] * (v * inv));
-    };
-    // The thread's y values, 4 consecutive elements per 1024-element block,
-    // read once and kept in registers (K <= 16384), or re-read below.
-    constexpr int NB = 16;
-    const bool held = K <= NB * 4 * WG;
     float yr[NB][4];
-    float amax = 0.f;
-    if (held) {
+    float ss = 0.f;
 #pragma unroll
-        for (int b = 0; b < NB; b++) {
-            const int base = b * 4 * WG + 4 * tid;
+    for (int b = 0; b < NB; b++) {
+        const int base = b * 4 * T + 4 * tid;   // K % 32 == 0: whole quads
+        const int64_t at = (int64_t)t * K + base;
+        FVec<4> v{};
+        if (base < K) {
+            if constexpr (SRC == SRC_ROW) {
+                v.load(a.x + at);
+            } else if constexpr (SRC == SRC_ADD) {
+                FVec<4> y;
+                y.load_parts(a.pa + at, a.nparts, a.stride);
+                v.load(a.x + at);
+                v.add(y);
+                v.store(a.x + at);
+            } else {
+                FVec<4> g, u;
+                g.load_parts(a.pa + at, a.nparts, a.stride);
+                u.load_parts(a.pb + at, a.nparts, a.stride);
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                yr[b][j] = base < K ? yval(base + j) : 0.f;   // K % 32 == 0: whole quads
-                amax = fmaxf(amax, fabsf(yr[b][j]));
+                for (int j = 0; j < 4; j++) {
+#pragma clang fp contract(off)
+                    // SiluInPlace then Mul (IE:463-474): ExpApprox on the vector lanes
+                    const float sg = base + j < n8 ? silu_ref(g.v[j]) : g.v[j] / (1.0f + expf(-g.v[j]));
+                    v.v[j] = sg * u.v[j];
+                }
             }
         }
-    } else {
-        for (int i = tid; i < K; i += WG) amax = fmaxf(amax, fabsf(yval(i)));
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            yr[b][j] = v.v[j];
+            if (NORM) ss += v.v[j] * v.v[j];
+        }
     }
+    if (NORM) {
+        ss = wave_sum(ss);
+        if (lane == 0) red[0][wave] = ss;
+        __syncthreads();
+        float tot = 0.f, inv;
+#pragma unroll
+        for (int i = 0; i < T / 64; i++) tot += red[0][i];
+        {
+#pragma clang fp contract(off)
+            inv = 1.0f / sqrtf((tot / (float)K) + a.eps);
+        }
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            const int base = b * 4 * T + 4 * tid;
+            FVec<4> w{};
+            if (base < K) w.load(a.w + base);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+#pragma clang fp contract(off)
+                yr[b][j] = base + j < n8 ? ((w.v[j] * yr[b][j]) * inv) : (w.v[j] * (yr[b][j] * inv));
+            }
+        }
+    }
+    float amax = 0.f;
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) amax = fmaxf(amax, fabsf(yr[b][j]));
     amax = wave_max(amax);
-    if (lane == 0) red[wave] = amax;
+    if (lane == 0) red[1][wave] = amax;
     __syncthreads();
     float m = 0.f;
 #pragma unroll
-    for (int i = 0; i < WG / 64; i++) m = fmaxf(m, red[i]);
+    for (int i = 0; i < T / 64; i++) m = fmaxf(m, red[1][i]);
     int e = 0;
     if (m > 0.f) {
         (void)frexpf(m, &e);          // m = f 2^e, f in [0.5, 1)
@@ -129,43 +216,30 @@ __global__ __launch_bounds__(WG) void pf_planes_kernel(const float* __restrict__
         e = e > 126 ? 126 : (e < -126 ? -126 : e);
     }
     const float s = ldexpf(1.0f, e), s32 = ldexpf(1.0f, e - 5);
-    if (tid == 0) xinv[t] = ldexpf(1.0f, -e);
+    if (tid == 0) a.p.xinv[t] = ldexpf(1.0f, -e);
     // 4 consecutive elements per thread; 8 threads cover one 32-element group
-    auto emit = [&](const int base, const float* y) __attribute__((always_inline)) {
-        float g = 0.f;
 #pragma unroll
-        for (int j = 0; j < 4; j++) g += y[j];
-        g = sum8(g);
+    for (int b = 0; b < NB; b++) {
+        const int base = b * 4 * T + 4 * tid;
+        if (b * 4 * T >= K) break;   // uniform: every lane calls sum8
+        const float g = sum8(((yr[b][0] + yr[b][1]) + yr[b][2]) + yr[b][3]);
         if (base < K) {
             h4 hv, lv;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const float ys = y[j] * s;
+                const float ys = yr[b][j] * s;
                 const _Float16 hi = (_Float16)ys;
                 hv[j] = hi;
                 lv[j] = (_Float16)(ys - (float)hi);
             }
-            *reinterpret_cast<h4*>(xh + (int64_t)t * K + base) = hv;
-            *reinterpret_cast<h4*>(xl + (int64_t)t * K + base) = lv;
+            *reinterpret_cast<h4*>(a.p.xh + (int64_t)t * K + base) = hv;
+            *reinterpret_cast<h4*>(a.p.xl + (int64_t)t * K + base) = lv;
             if ((tid & 7) == 0) {
                 const float gs = g * s32;
                 const _Float16 hi = (_Float16)gs;
-                sh[(int64_t)t * (K / 32) + base / 32] = hi;
-                sl[(int64_t)t * (K / 32) + base / 32] = (_Float16)(gs - (float)hi);
+                a.p.sh[(int64_t)t * (K / 32) + base / 32] = hi;
+                a.p.sl[(int64_t)t * (K / 32) + base / 32] = (_Float16)(gs - (float)hi);
             }
-        }
-    };
-    if (held) {
-#pragma unroll
-        for (int b = 0; b < NB; b++)
-            if (b * 4 * WG < K) emit(b * 4 * WG + 4 * tid, yr[b]);   // uniform: every lane calls sum8
-    } else {
-        for (int b0 = 0; b0 < K; b0 += 4 * WG) {
-            const int base = b0 + 4 * tid;
-            float y[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) y[j] = base < K ? yval(base + j) : 0.f;
-            emit(base, y);
         }
     }
 }
@@ -187,6 +261,7 @@ struct PfGemmArgs {
     const uint8_t* wb;
     float* outb;
     int tn_b, nb, ldob;
+    int64_t part_stride_b;
 };
 
 __device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) {
@@ -220,7 +295,7 @@ __device__ __forceinline__ uint32_t k_field12(uint32_t w1, uint32_t w2, uint32_t
 // rows touches 256 contiguous bytes); the 2-byte aligned formats copy windows
 // starting at the block address rounded down to 4 bytes ([row][ch]).
 // Every step's partial sum is scaled by the row's block scale d; NP = weight
-// planes; NS = LDS stages (prefetch distance NS - 1).  RH > 0: the weights
+// planes.  RH > 0: the weights
 // are staged once per 4 steps instead, RH chunks per row.  Q6_K: the 4 steps
 // of a half superblock read the same qh bytes and pairs of them the same ql
 // bytes, which a per-step copy fetched again each time (128 bytes per row and
@@ -229,15 +304,15 @@ __device__ __forceinline__ uint32_t k_field12(uint32_t w1, uint32_t w2, uint32_t
 template <uint32_t FMT>
 struct PfFmt;
 template <>
-struct PfFmt<GGML_Q4_K> { static constexpr int BSZ = 144, EPB = 256, R = 2, NP = 1, NS = 2, RH = 0; static constexpr bool MIN = true, KQ = true; };
+struct PfFmt<GGML_Q4_K> { static constexpr int BSZ = 144, EPB = 256, R = 2, NP = 1, RH = 0; static constexpr bool MIN = true, KQ = true; };
 template <>
-struct PfFmt<GGML_Q5_K> { static constexpr int BSZ = 176, EPB = 256, R = 4, NP = 1, NS = 2, RH = 0; static constexpr bool MIN = true, KQ = true; };
+struct PfFmt<GGML_Q5_K> { static constexpr int BSZ = 176, EPB = 256, R = 4, NP = 1, RH = 0; static constexpr bool MIN = true, KQ = true; };
 template <>
-struct PfFmt<GGML_Q6_K> { static constexpr int BSZ = 210, EPB = 256, R = 8, NP = 2, NS = 2, RH = 10; static constexpr bool MIN = false, KQ = false; };
+struct PfFmt<GGML_Q6_K> { static constexpr int BSZ = 210, EPB = 256, R = 8, NP = 2, RH = 10; static constexpr bool MIN = false, KQ = false; };
 template <>
-struct PfFmt<GGML_Q8_0> { static constexpr int BSZ = 34, EPB = 32, R = 4, NP = 1, NS = 2, RH = 10; static constexpr bool MIN = false, KQ = false; };
+struct PfFmt<GGML_Q8_0> { static constexpr int BSZ = 34, EPB = 32, R = 4, NP = 1, RH = 10; static constexpr bool MIN = false, KQ = false; };
 template <>
-struct PfFmt<GGML_Q4_0> { static constexpr int BSZ = 18, EPB = 32, R = 2, NP = 1, NS = 2, RH = 0; static constexpr bool MIN = false, KQ = false; };
+struct PfFmt<GGML_Q4_0> { static constexpr int BSZ = 18, EPB = 32, R = 2, NP = 1, RH = 0; static constexpr bool MIN = false, KQ = false; };
 
 // K-quants: byte offset of chunk ch of group g within a superblock.
 template <uint32_t FMT>
@@ -398,20 +473,37 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // conflict-free to read, made the copies slower than it saved).
 __device__ __forceinline__ int swz(int r) { return (r >> 1) & 3; }
 
-// TM tokens per workgroup: BM, or 64 for launches that would have only 128
-// to 255 tiles of BM (all CUs busy; each output's sum runs in the same order).
+// LDS stages (copies run NS - 1 steps ahead) for TM-token tiles.
+constexpr int gemm_stages(int tm) { return tm == BM ? 2 : tm == 64 ? 3 : 4; }
+
+// Waits for the oldest of the copies in flight: those of `later` more steps
+// may remain, each at least N instructions of this wave.
+template <int N>
+__device__ __forceinline__ void wait_steps(int later) {
+    if (later >= 2) vm_wait<2 * N>();
+    else if (later == 1) vm_wait<N>();
+    else vm_wait<0>();
+}
+
+// TM tokens per workgroup (each output's sum runs in the same order for all):
+// 128 where the launch fills the chip, 64 and 32 where tokens are few
+// (prefill_plan).  A 128-token tile is bound by its chain per step (copy wait,
+// barrier, fragments, MFMAs) at two workgroups a CU; a 32-token one has a
+// quarter of the MFMAs and is bound by the copies' latency, so it keeps three
+// steps in flight, and its registers and LDS allow 3-4 workgroups a CU.
 template <uint32_t FMT, int EPI, int TM = BM>
-__global__ __launch_bounds__(WG, 2) void pf_gemm_kernel(PfGemmArgs a) {
+__global__ __launch_bounds__(WG, TM == 32 ? 4 : 2) void pf_gemm_kernel(PfGemmArgs a) {
     using F = PfFmt<FMT>;
-    static_assert(TM == BM || (TM == 64 && EPI != PF_SWIGLU), "64-token tiles: STORE and ADD only");
-    constexpr int NP = F::NP, R = F::R, NS = F::NS;
+    static_assert(TM == BM || ((TM == 64 || TM == 32) && EPI != PF_SWIGLU), "small tiles: STORE and ADD only");
+    constexpr int NP = F::NP, R = F::R, NS = gemm_stages(TM);
+    constexpr int TS = TM < 64 ? 64 : TM;            // tokens per plane of the group sums (a whole copy)
     constexpr int TI = TM / 16, TJ = BN / 16 / 4;    // wave w: all TM tokens x rows 16 TJ w .. +16 TJ - 1
     constexpr bool WH = F::RH > 0;                   // weights staged once per 4 steps
     constexpr int XS1 = 2 * TM * 64;                 // activation stage: [plane][token][32 halves]
     constexpr int WS1 = WH ? 0 : BN * R * 16;        // raw weight stage (per step)
     constexpr int WSH = WH ? BN * F::RH * 16 : 0;    // raw weight stage (per 4 steps), two of them
     constexpr int ST1 = XS1 + WS1;
-    constexpr int SS_B = F::MIN ? 2 * 2 * TM * 16 : 0;   // [sb parity][plane][token][8] group sums
+    constexpr int SS_B = F::MIN ? 2 * 2 * TS * 16 : 0;   // [sb parity][plane][token][8] group sums
     constexpr int STAGE_B = NS * ST1 + SS_B + 2 * WSH;
     constexpr int EX_B = 2 * TM * (16 * TJ + 1) * 4;     // SWIGLU exchange: [gate wave][token][rows + 1]
     constexpr int SMEM = STAGE_B > EX_B ? STAGE_B : EX_B;
@@ -434,8 +526,11 @@ __global__ __launch_bounds__(WG, 2) void pf_gemm_kernel(PfGemmArgs a) {
     const int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
     if (tile >= ntm * ntn * a.ksplit) return;
     const int tn = tile % ntn, m0 = ((tile / ntn) % ntm) * TM, part = tile / (ntn * ntm);
-    const int K = a.K, spp = K / 32 / a.ksplit;   // 32-element steps per part
-    const int st0 = part * spp, st1 = st0 + spp;
+    // K parts: units of whole superblocks (of 4 steps for the 32-element
+    // blocks), dealt out evenly
+    constexpr int UNIT = F::EPB == 256 ? 8 : 4;
+    const int K = a.K, units = (K / 32 + UNIT - 1) / UNIT;
+    const int st0 = units * part / a.ksplit * UNIT, st1 = min(units * (part + 1) / a.ksplit * UNIT, K / 32);
     const int64_t rbytes = (int64_t)(K / F::EPB) * F::BSZ;
     // the matrix this row tile reads (uniform per workgroup): the second one
     // from row tile tn_b on
@@ -470,7 +565,7 @@ __global__ __launch_bounds__(WG, 2) void pf_gemm_kernel(PfGemmArgs a) {
         woff[j] = (uint32_t)wrow[j];
     }
     uint32_t soff = 0;
-    if (F::MIN) soff = (uint32_t)((int64_t)min(m0 + ((wv * 64 + lane) & (TM - 1)), a.M - 1) * (K / 32) * 2);
+    if (F::MIN) soff = (uint32_t)((int64_t)min(m0 + ((wv * 64 + lane) & (TS - 1)), a.M - 1) * (K / 32) * 2);
 
     auto issue = [&](int st) __attribute__((always_inline)) {
         const uint32_t lb = sm + (uint32_t)((st % NS) * ST1);
@@ -505,9 +600,9 @@ __global__ __launch_bounds__(WG, 2) void pf_gemm_kernel(PfGemmArgs a) {
                 dma16(wsel(q0 / R), o, lb + XS1 + (NW * wv + j) * 1024);
             }
         }
-        if (F::MIN && (st & 7) == 0 && wv < TM / 32) {   // TM / 32 x 1 KB of group sums
-            const char* sbase = reinterpret_cast<const char*>(wv >= TM / 64 ? a.sl : a.sh) + 16 * (st >> 3);
-            dma16(sbase, soff, sm + (uint32_t)(NS * ST1 + ((st >> 3) & 1) * (2 * TM * 16) + wv * 1024));
+        if (F::MIN && (st & 7) == 0 && wv < TS / 32) {   // TS / 32 x 1 KB of group sums
+            const char* sbase = reinterpret_cast<const char*>(wv >= TS / 64 ? a.sl : a.sh) + 16 * (st >> 3);
+            dma16(sbase, soff, sm + (uint32_t)(NS * ST1 + ((st >> 3) & 1) * (2 * TS * 16) + wv * 1024));
         }
     };
     // fragment addresses: activation rows ti * 16 + lr, weight rows rw[tj]
@@ -532,16 +627,17 @@ __global__ __launch_bounds__(WG, 2) void pf_gemm_kernel(PfGemmArgs a) {
 #pragma unroll
     for (int j = 0; j < TJ; j++) hdr[j] = v4u{0u, 0u, 0u, 0u};
 
-    issue(st0);
-    if (NS == 3 && st0 + 1 < st1) issue(st0 + 1);
+    // copies a step brings at least: the activations', and the weights' except
+    // a header chunk's (superblocks' first steps only) or a 4-step stage's
+    constexpr int LB = NX + (WH ? 0 : NW);
+    const bool header_wave = F::KQ && ((NW * wv * 64) >> 7) == 0;
+#pragma unroll
+    for (int i = 0; i < NS - 1; i++)
+        if (st0 + i < st1) issue(st0 + i);
     for (int st = st0; st < st1; st++) {
-        // step st's copies are complete once at most the later step's remain
-        if (NS == 3 && st + 1 < st1) {
-            if (F::MIN && ((st + 1) & 7) == 0) vm_wait<NX + NW + 1>();
-            else vm_wait<NX + NW>();
-        } else {
-            vm_wait<0>();
-        }
+        const int later = min(NS - 2, st1 - 1 - st);
+        if (header_wave) wait_steps<NX>(later);
+        else wait_steps<LB>(later);
         lds_barrier();   // every wave's copies of step st landed; step st - 1's buffers are free
         if (st + NS - 1 < st1) issue(st + NS - 1);
         const unsigned char* sb = smem + (st % NS) * ST1;
@@ -617,8 +713,8 @@ __global__ __launch_bounds__(WG, 2) void pf_gemm_kernel(PfGemmArgs a) {
                         const int tl = ti * 16 + lr;
                         h4 s0 = h4{0, 0, 0, 0}, s1 = h4{0, 0, 0, 0};
                         if (lk < 2) {
-                            s0 = *reinterpret_cast<const h4*>(Ss + ((sp * 2 + 0) * TM + tl) * 16 + 8 * lk);
-                            s1 = *reinterpret_cast<const h4*>(Ss + ((sp * 2 + 1) * TM + tl) * 16 + 8 * lk);
+                            s0 = *reinterpret_cast<const h4*>(Ss + ((sp * 2 + 0) * TS + tl) * 16 + 8 * lk);
+                            s1 = *reinterpret_cast<const h4*>(Ss + ((sp * 2 + 1) * TS + tl) * 16 + 8 * lk);
                         }
                         f4 rr = __builtin_amdgcn_mfma_f32_16x16x16f16(s0, mq, f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
                         rr = __builtin_amdgcn_mfma_f32_16x16x16f16(s1, mq, rr, 0, 0, 0);
@@ -687,7 +783,7 @@ __global__ __launch_bounds__(WG, 2) void pf_gemm_kernel(PfGemmArgs a) {
                     const int row = tnl * BN + wn * 16 * TJ + tj * 16 + lr;
                     if (t < a.M && row < Nl) {
                         const float y = acc[ti][tj][e] * xi[ti][e];
-                        float* o = segb ? a.outb + (int64_t)t * a.ldob + row
+                        float* o = segb ? a.outb + part * a.part_stride_b + (int64_t)t * a.ldob + row
                                         : a.out + part * a.part_stride + (int64_t)t * a.ldo + row;
                         if (EPI == PF_ADD) {
 #pragma clang fp contract(off)
@@ -711,57 +807,6 @@ __device__ __forceinline__ float sum_parts(const float* x, int64_t idx, int n, i
     for (int p = 1; p < n; p++) v += x[p * stride + idx];
     return v;
 }
-
-template <int V>
-struct FVec {
-    float v[V];
-    __device__ __forceinline__ void load(const float* p) {
-        if constexpr (V == 4) {
-            const f4 x = *reinterpret_cast<const f4*>(p);
-#pragma unroll
-            for (int i = 0; i < 4; i++) v[i] = x[i];
-        } else {
-            v[0] = p[0];
-        }
-    }
-    // parts in order, four of them in flight
-    __device__ __forceinline__ void load_parts(const float* x, int n, int64_t stride) {
-        load(x);
-        int p = 1;
-        for (; p + 3 < n; p += 4) {
-            FVec t[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) t[j].load(x + (p + j) * stride);
-#pragma unroll
-            for (int j = 0; j < 4; j++) add(t[j]);
-        }
-        for (; p < n; p++) {
-            FVec t;
-            t.load(x + p * stride);
-            add(t);
-        }
-    }
-    __device__ __forceinline__ void add(const FVec& o) {
-#pragma unroll
-        for (int i = 0; i < V; i++) v[i] += o.v[i];
-    }
-    __device__ __forceinline__ void store(float* p) const {
-        if constexpr (V == 4) *reinterpret_cast<f4*>(p) = f4{v[0], v[1], v[2], v[3]};
-        else p[0] = v[0];
-    }
-    __device__ __forceinline__ void store_kv(void* cache, int64_t idx, int fp16) const {
-        if constexpr (V == 4) {
-            if (fp16) {
-                *reinterpret_cast<h4*>(reinterpret_cast<_Float16*>(cache) + idx) =
-                    h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-            } else {
-                store(reinterpret_cast<float*>(cache) + idx);
-            }
-        } else {
-            llmdot::store_kv(cache, idx, v[0], fp16);
-        }
-    }
-};
 
 // Models without per-head norms.  A thread takes V rotation pairs (or 2 V
 // elements that do not rotate) of one head of one token: elements i .. i+V-1
@@ -880,15 +925,23 @@ __global__ __launch_bounds__(WG) void pf_rope_kv_kernel(PfAttnArgs a) {
     }
 }
 
-// h[i] += parts[0][i] + parts[1][i] + ... (in part order) for i < n: the
-// residual add of an output projection computed in K parts.
-__global__ __launch_bounds__(WG) void pf_add_parts_kernel(float* __restrict__ h, const float* __restrict__ parts,
+// y[i] = parts[0][i] + parts[1][i] + ... (in part order), added to out or
+// stored, for i < n in groups of V.
+template <bool ADD, int V>
+__global__ __launch_bounds__(WG) void pf_sum_parts_kernel(float* __restrict__ out, const float* __restrict__ parts,
                                                           int nparts, int64_t stride, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x;
+    const int64_t i = ((int64_t)blockIdx.x * WG + threadIdx.x) * V;
     if (i >= n) return;
-    float y = parts[i];
-    for (int p = 1; p < nparts; p++) y += parts[p * stride + i];
-    h[i] += y;
+    FVec<V> y;
+    y.load_parts(parts + i, nparts, stride);
+    if (ADD) {
+        FVec<V> h;
+        h.load(out + i);
+        h.add(y);
+        h.store(out + i);
+    } else {
+        y.store(out + i);
+    }
 }
 
 // ------------------------------------------------------------- attention --
@@ -1156,25 +1209,20 @@ __global__ __launch_bounds__(WG, 3) void pf_attn_pv_mfma(PfAttnArgs a) {
 }
 
 template <uint32_t FMT>
-hipError_t launch_gemm_fmt(int epi, PfGemmArgs a, hipStream_t s) {
+hipError_t launch_gemm_fmt(int epi, PfGemmArgs a, int tm, hipStream_t s) {
     const int tn_a = epi == PF_SWIGLU ? (a.N + 63) / 64 : (a.N + BN - 1) / BN;
     a.tiles_n = tn_a + (a.wb ? (a.nb + BN - 1) / BN : 0);
     a.tn_b = tn_a;
-    const int tiles = a.tiles_n * ((a.M + BM - 1) / BM) * a.ksplit;
-    // 128 to 255 tiles of BM tokens fill only part of the CUs: 64-token tiles
-    // (LLMDOT_HIP_PF_TM64=0 turns this off)
-    const char* env = getenv("LLMDOT_HIP_PF_TM64");
-    const bool tm64_off = env && env[0] == '0' && env[1] == 0;
-    const bool tm64 = !tm64_off && epi != PF_SWIGLU && a.ksplit == 1 && tiles >= 128 && tiles < 256;
-    const int t64 = a.tiles_n * ((a.M + 63) / 64);
-    const dim3 grid(8 * (((tm64 ? t64 : tiles) + 7) / 8));
+    const int tiles = a.tiles_n * ((a.M + tm - 1) / tm) * a.ksplit;
+    const dim3 grid(8 * ((tiles + 7) / 8));
     switch (epi) {
     case PF_STORE:
-        if (tm64) pf_gemm_kernel<FMT, PF_STORE, 64><<<grid, WG, 0, s>>>(a);
+        if (tm == 32) pf_gemm_kernel<FMT, PF_STORE, 32><<<grid, WG, 0, s>>>(a);
+        else if (tm == 64) pf_gemm_kernel<FMT, PF_STORE, 64><<<grid, WG, 0, s>>>(a);
         else pf_gemm_kernel<FMT, PF_STORE><<<grid, WG, 0, s>>>(a);
         break;
     case PF_ADD:
-        if (tm64) pf_gemm_kernel<FMT, PF_ADD, 64><<<grid, WG, 0, s>>>(a);
+        if (tm == 64) pf_gemm_kernel<FMT, PF_ADD, 64><<<grid, WG, 0, s>>>(a);
         else pf_gemm_kernel<FMT, PF_ADD><<<grid, WG, 0, s>>>(a);
         break;
     case PF_SWIGLU: pf_gemm_kernel<FMT, PF_SWIGLU><<<grid, WG, 0, s>>>(a); break;
@@ -1203,53 +1251,75 @@ bool prefill_gemm_supported(uint32_t type, int cols) {
     }
 }
 
-hipError_t launch_prefill_planes(const float* x, int M, int K, const float* norm_w, float eps, const PfPlanes& p,
-                                 hipStream_t s) {
-    if (M <= 0 || K <= 0 || K % 32) return hipErrorInvalidValue;
-    if (norm_w) pf_planes_kernel<true><<<M, WG, 0, s>>>(x, K, norm_w, eps, p.xh, p.xl, p.sh, p.sl, p.xinv);
-    else pf_planes_kernel<false><<<M, WG, 0, s>>>(x, K, nullptr, eps, p.xh, p.xl, p.sh, p.sl, p.xinv);
-    return hipGetLastError();
-}
-
 namespace {
-hipError_t launch_gemm_type(uint32_t type, int epi, const PfGemmArgs& a, hipStream_t s) {
-    switch (type) {
-    case GGML_Q4_K: return launch_gemm_fmt<GGML_Q4_K>(epi, a, s);
-    case GGML_Q5_K: return launch_gemm_fmt<GGML_Q5_K>(epi, a, s);
-    case GGML_Q6_K: return launch_gemm_fmt<GGML_Q6_K>(epi, a, s);
-    case GGML_Q8_0: return launch_gemm_fmt<GGML_Q8_0>(epi, a, s);
-    case GGML_Q4_0: return launch_gemm_fmt<GGML_Q4_0>(epi, a, s);
-    default: return hipErrorInvalidValue;
+template <bool NORM, int SRC>
+hipError_t launch_planes(const PfPlanesArgs& a, int M, hipStream_t s) {
+    if (M <= 0 || a.K <= 0 || a.K % 32 || a.K > 16384) return hipErrorInvalidValue;
+    if (M <= 256) {
+        if (a.K <= 4096) pf_planes_kernel<NORM, SRC, 1, 1024><<<M, 1024, 0, s>>>(a);
+        else pf_planes_kernel<NORM, SRC, 4, 1024><<<M, 1024, 0, s>>>(a);
+    } else {
+        if (a.K <= 4096) pf_planes_kernel<NORM, SRC, 4, WG><<<M, WG, 0, s>>>(a);
+        else pf_planes_kernel<NORM, SRC, 16, WG><<<M, WG, 0, s>>>(a);
     }
+    return hipGetLastError();
 }
 }  // namespace
 
-hipError_t launch_prefill_gemm(uint32_t type, int epi, const PfPlanes& p, const uint8_t* w, const uint8_t* w2, int M,
-                               int N, int K, float* out, int ldo, hipStream_t s, int ksplit, int64_t part_stride) {
-    if (M <= 0 || N <= 0 || !prefill_gemm_supported(type, K) || (epi == PF_SWIGLU && !w2) || ldo < N)
-        return hipErrorInvalidValue;
-    // parts of whole blocks (256-element superblocks for the K-quants), STORE only
-    const int gran = block_elems(type) == 256 ? 8 : 1;
-    if (ksplit < 1 || (ksplit > 1 && (epi != PF_STORE || (K / 32) % (ksplit * gran) != 0 ||
-                                      part_stride < (int64_t)(M - 1) * ldo + N)))
-        return hipErrorInvalidValue;
-    // the kernel addresses activations and weight rows with 32-bit byte offsets
-    if ((int64_t)M * K * 2 >= (int64_t)1 << 31 || (int64_t)N * byte_count(type, K) >= ((int64_t)1 << 31) - 65536)
-        return hipErrorInvalidValue;
-    PfGemmArgs a{p.xh, p.xl, p.sh, p.sl, p.xinv, w, w2, out, M, N, K, ldo, 0, ksplit, part_stride};
-    return launch_gemm_type(type, epi, a, s);
+hipError_t launch_prefill_planes(const float* x, int M, int K, const float* norm_w, float eps, const PfPlanes& p,
+                                 hipStream_t s) {
+    const PfPlanesArgs a{const_cast<float*>(x), nullptr, nullptr, 0, 0, K, norm_w, eps, p};
+    return norm_w ? launch_planes<true, SRC_ROW>(a, M, s) : launch_planes<false, SRC_ROW>(a, M, s);
 }
 
-hipError_t launch_prefill_gemm_pair(uint32_t type, const PfPlanes& p, const uint8_t* w, int N, float* out, int ldo,
-                                    const uint8_t* wb, int nb, float* outb, int ldob, int M, int K, hipStream_t s) {
-    if (M <= 0 || N <= 0 || nb <= 0 || N % BN || !w || !wb || !prefill_gemm_supported(type, K) || ldo < N ||
-        ldob < nb)
+hipError_t launch_prefill_planes_add(float* h, const float* parts, int nparts, int64_t stride, int M, int K,
+                                     const float* norm_w, float eps, const PfPlanes& p, hipStream_t s) {
+    if (nparts < 1 || stride % 4 || !norm_w) return hipErrorInvalidValue;
+    return launch_planes<true, SRC_ADD>(PfPlanesArgs{h, parts, nullptr, nparts, stride, K, norm_w, eps, p}, M, s);
+}
+
+hipError_t launch_prefill_planes_swiglu(const float* gate, const float* up, int nparts, int64_t stride, int M, int K,
+                                        const PfPlanes& p, hipStream_t s) {
+    if (nparts < 1 || stride % 4) return hipErrorInvalidValue;
+    return launch_planes<false, SRC_SWIGLU>(PfPlanesArgs{nullptr, gate, up, nparts, stride, K, nullptr, 0.f, p}, M, s);
+}
+
+namespace {
+hipError_t launch_gemm_type(uint32_t type, int epi, const PfGemmArgs& a, int tm, hipStream_t s) {
+    switch (type) {
+    case GGML_Q4_K: return launch_gemm_fmt<GGML_Q4_K>(epi, a, tm, s);
+    case GGML_Q5_K: return launch_gemm_fmt<GGML_Q5_K>(epi, a, tm, s);
+    case GGML_Q6_K: return launch_gemm_fmt<GGML_Q6_K>(epi, a, tm, s);
+    case GGML_Q8_0: return launch_gemm_fmt<GGML_Q8_0>(epi, a, tm, s);
+    case GGML_Q4_0: return launch_gemm_fmt<GGML_Q4_0>(epi, a, tm, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+// K part units (see pf_gemm_kernel)
+int gemm_units(uint32_t type, int K) { return block_elems(type) == 256 ? K / 256 : (K / 32 + 3) / 4; }
+}  // namespace
+
+hipError_t launch_prefill_gemm(uint32_t type, int epi, const PfPlanes& p, const PfMat& wa, const PfMat& wb, int M,
+                               int K, const PfPlan& plan, hipStream_t s) {
+    if (M <= 0 || wa.rows <= 0 || !wa.w || !wa.out || !prefill_gemm_supported(type, K) || wa.ld < wa.rows)
         return hipErrorInvalidValue;
+    if (wb.w && (epi == PF_ADD || wb.rows <= 0)) return hipErrorInvalidValue;
+    if (epi == PF_SWIGLU && (!wb.w || wb.rows != wa.rows)) return hipErrorInvalidValue;
+    const bool pair = epi == PF_STORE && wb.w;
+    if (pair && (wa.rows % BN || !wb.out || wb.ld < wb.rows)) return hipErrorInvalidValue;
+    const bool tm_ok = plan.tm == BM || (plan.tm == 64 && epi != PF_SWIGLU) || (plan.tm == 32 && epi == PF_STORE);
+    if (!tm_ok || plan.ksplit < 1 || plan.ksplit > gemm_units(type, K)) return hipErrorInvalidValue;
+    if (plan.ksplit > 1 && (epi != PF_STORE || wa.part_stride < (int64_t)(M - 1) * wa.ld + wa.rows ||
+                            (pair && wb.part_stride < (int64_t)(M - 1) * wb.ld + wb.rows)))
+        return hipErrorInvalidValue;
+    // the kernel addresses activations and weight rows with 32-bit byte offsets
     if ((int64_t)M * K * 2 >= (int64_t)1 << 31 ||
-        (int64_t)std::max(N, nb) * byte_count(type, K) >= ((int64_t)1 << 31) - 65536)
+        (int64_t)std::max(wa.rows, wb.w ? wb.rows : 0) * byte_count(type, K) >= ((int64_t)1 << 31) - 65536)
         return hipErrorInvalidValue;
-    PfGemmArgs a{p.xh, p.xl, p.sh, p.sl, p.xinv, w, nullptr, out, M, N, K, ldo, 0, 1, 0, wb, outb, 0, nb, ldob};
-    return launch_gemm_type(type, PF_STORE, a, s);
+    PfGemmArgs a{p.xh, p.xl, p.sh, p.sl, p.xinv, wa.w, epi == PF_SWIGLU ? wb.w : nullptr, wa.out, M, wa.rows, K, wa.ld,
+                 0, plan.ksplit, wa.part_stride};
+    if (pair) { a.wb = wb.w; a.outb = wb.out; a.nb = wb.rows; a.ldob = wb.ld; a.part_stride_b = wb.part_stride; }
+    return launch_gemm_type(type, epi, a, plan.tm, s);
 }
 
 hipError_t launch_prefill_rope_kv(const PfAttnArgs& a, hipStream_t s) {
@@ -1268,19 +1338,74 @@ hipError_t launch_prefill_rope_kv(const PfAttnArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_prefill_add_parts(float* h, const float* parts, int nparts, int64_t stride, int64_t n, hipStream_t s) {
+hipError_t launch_prefill_sum_parts(float* out, bool add, const float* parts, int nparts, int64_t stride, int64_t n,
+                                    hipStream_t s) {
     if (n <= 0 || nparts < 1 || stride < n) return hipErrorInvalidValue;
-    pf_add_parts_kernel<<<(unsigned)((n + WG - 1) / WG), WG, 0, s>>>(h, parts, nparts, stride, n);
+    const bool v4 = n % 4 == 0 && stride % 4 == 0;
+    const int64_t items = v4 ? n / 4 : n;
+    const unsigned grid = (unsigned)((items + WG - 1) / WG);
+    if (v4 && add) pf_sum_parts_kernel<true, 4><<<grid, WG, 0, s>>>(out, parts, nparts, stride, n);
+    else if (v4) pf_sum_parts_kernel<false, 4><<<grid, WG, 0, s>>>(out, parts, nparts, stride, n);
+    else if (add) pf_sum_parts_kernel<true, 1><<<grid, WG, 0, s>>>(out, parts, nparts, stride, n);
+    else pf_sum_parts_kernel<false, 1><<<grid, WG, 0, s>>>(out, parts, nparts, stride, n);
     return hipGetLastError();
 }
 
-int prefill_ksplit(uint32_t type, int M, int N, int K) {
-    const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-    const int gran = block_elems(type) == 256 ? 8 : 1;
-    int sp = 1;
-    if (tiles >= 128) return 1;
-    while (sp < 8 && tiles * sp * 2 <= 512 && (K / 32) % (sp * 2 * gran) == 0) sp *= 2;
-    return sp;
+namespace {
+// Estimated microseconds of a STORE launch, from measured rates per tile
+// height: a workgroup alone on its CU takes `alone` per 32-column step (a chain
+// of copy wait, barrier, fragments and MFMAs), two on a CU `two` per step of
+// both (launches of 257 to 511 workgroups have some of each), and a CU with more
+// `full` per workgroup and step; a workgroup's start and end cost about 10
+// steps.  Parts are written and read back at about 4 TB/s.  Measured (us; tile
+// height and K parts): Q4_K 23 x 28672 x 4096: 128-token tiles 103, 32-token
+// 65, in 4 parts 39; 23 x 4096 x 14336: 332, 218, in 16 parts 24; 64 x 28672 x
+// 4096: 128-token tiles 107, 64-token 83, in 2 parts 57; 512 x 2048 x 8192:
+// 199, in 8 parts 49; 256 x 28672 x 4096 (448 tiles): 154 in any split; Q6_K
+// 777 x 3072 x 8192 (168 tiles): 238, in 3 parts 128, 64-token tiles 222, 167.
+double gemm_us(int tm, int M, int N, int steps, double parts, int sp) {
+    const double alone = tm == 32 ? 0.47 : tm == 64 ? 0.58 : 0.80;
+    const double two = tm == 32 ? 0.58 : tm == 64 ? 0.77 : 1.15;
+    const double full = tm == 32 ? 0.27 : tm == 64 ? 0.42 : 0.65;
+    const double load = (double)((M + tm - 1) / tm) * ((N + BN - 1) / BN) * sp / 256;   // workgroups per CU
+    const double step = load <= 1 ? alone : load <= 2 ? alone + (two - alone) * (load - 1) : std::max(two, load * full);
+    return (steps + 10) * step + parts * M * N * 4.0 / 4e6;
+}
+
+// The cheapest tile and split; the parts hold at most max_parts floats.
+// always_parts: the results go through a parts buffer unsplit too.
+PfPlan best_plan(uint32_t type, int M, int N, int K, int64_t max_parts, bool always_parts, double* us) {
+    const int units = gemm_units(type, K), unit = block_elems(type) == 256 ? 8 : 4;
+    const bool no64 = [] { const char* e = getenv("LLMDOT_HIP_PF_TM64"); return e && e[0] == '0' && e[1] == 0; }();
+    PfPlan best{BM, 1};
+    *us = 1e30;
+    for (int tm : {128, 64, 32}) {
+        // smaller tiles dequantise each weight once per tile: 32 tokens only
+        // where one tile holds them all (301 x 5632 x 1024 Q5_K: 33 us against
+        // 24 with 64 in 2 parts), 64 never where the chip is full
+        if (tm == 32 ? M > 32 : tm == 64 && M > 1024) continue;
+        for (int sp = 1; sp <= std::min(16, units); sp++) {
+            if ((sp > 1 || always_parts) && (int64_t)sp * M * N > max_parts) break;
+            const double t = gemm_us(tm, M, N, (units + sp - 1) / sp * unit, sp > 1 || always_parts ? sp : 0, sp);
+            if (t < *us) { *us = t; best = {tm, sp}; }
+        }
+    }
+    if (no64 && best.tm == 64) best.tm = BM;
+    return best;
+}
+}  // namespace
+
+PfPlan prefill_plan(uint32_t type, int M, int N, int K, int64_t max_parts) {
+    double us;
+    return best_plan(type, M, N, K, max_parts, false, &us);
+}
+
+PfPlan prefill_swiglu_plan(uint32_t type, int M, int N, int K, int64_t max_parts) {
+    // one launch of 64 + 64 row tiles, the product written once and read by the planes
+    const double fused = gemm_us(BM, M, 2 * N, K / 32, 0.5, 1);
+    double us;
+    const PfPlan p = best_plan(type, M, 2 * N, K, 2 * max_parts, true, &us);
+    return us < fused ? p : PfPlan{BM, 1};
 }
 
 hipError_t launch_prefill_attention(const PfAttnArgs& a, hipStream_t s) {

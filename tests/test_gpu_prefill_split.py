@@ -7,8 +7,9 @@ Bounds: those of test_gpu_prefill.py (`_prompt_check`).
 import numpy as np
 import pytest
 
-from dotllm_amd import synth
-from test_gpu_prefill import _prompt_check, oracle_threads  # noqa: F401
+from dotllm_amd import Q4_0, Q4_K, Q5_K, Q6_K, Q8_0, synth
+from oracle import oracle as O
+from test_gpu_prefill import FP32_LEVEL, _prompt_check, oracle_threads, random_blocks, row_rel_err  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +43,17 @@ def test_prefill_attention_512_queries_groups(hip, oracle_threads):  # noqa: F81
     spec = dict(synth.SPECS["small5"], layers=1)
     img = synth.build_image("small5", seed=1234, spec=spec, context=600)
     _prompt_check(hip, img, synth.prompt(32000, 530, seed=7), 600, False, [0])
+
+
+@pytest.mark.parametrize("t,k", [(Q4_K, 2816), (Q5_K, 256), (Q6_K, 1280), (Q8_0, 1408), (Q8_0, 32), (Q4_0, 4192)])
+@pytest.mark.parametrize("m,n", [(2, 129), (32, 300), (33, 96), (64, 2000), (65, 128), (140, 520)])
+def test_batched_matmul_tiles_and_parts(hip, t, k, m, n):
+    """Edges of the 32-, 64- and 128-token tiles; K in uneven parts, one unit
+    only, and a last unit of fewer than 4 blocks."""
+    rng = np.random.default_rng(m + n + k)
+    w = random_blocks(t, n, k, m + n)
+    a = rng.normal(0, 1, size=(m, k)).astype(np.float32)
+    ref = O.matmul(a, w, t, k, n, result_len=m * n).reshape(m, n)
+    y = np.zeros(m * n, dtype=np.float32)
+    hip.mat_mul(a.reshape(-1), w, y, t, k, n)
+    assert row_rel_err(y.reshape(m, n), ref) <= FP32_LEVEL
