@@ -102,6 +102,12 @@ struct llmdot_hip_ctx {
     // two more streams (default priority) for independent prompt GEMMs, forked
     // from and joined back into `stream` with events
     hipStream_t side[2] = {nullptr, nullptr};
+    // Pinned host memory that a call's small inputs and results pass through
+    // (BOUNCE_BYTES; null: not available): copied by the host on one side, by a
+    // kernel on the stream on the other.  Every pageable copy of the runtime is
+    // a wait of its own, 10-20 us however small; a decode step made three.
+    uint8_t* bounce = nullptr;
+    size_t bounce_used = 0;
     hipEvent_t fork = nullptr, join[2] = {nullptr, nullptr};
     // models created on this context and not yet destroyed; llmdot_hip_destroy
     // with models alive defers the release to the last model's destroy
@@ -120,8 +126,31 @@ struct llmdot_hip_ctx {
 
 namespace {
 
+// Starts a call: its device, and all of the bounce memory.
 int ensure_device(llmdot_hip_ctx* ctx) {
     HIPCHK(hipSetDevice(ctx->device));
+    ctx->bounce_used = 0;
+    return 0;
+}
+
+constexpr size_t BOUNCE_BYTES = 1 << 20;
+
+// n bytes of the bounce memory for the rest of this call; null if they do not fit.
+uint8_t* bounce_take(llmdot_hip_ctx* ctx, size_t n) {
+    if (!ctx->bounce || n > BOUNCE_BYTES - ctx->bounce_used) return nullptr;
+    uint8_t* p = ctx->bounce + ctx->bounce_used;
+    ctx->bounce_used = std::min(BOUNCE_BYTES, (ctx->bounce_used + n + 255) & ~size_t(255));
+    return p;
+}
+
+// Host bytes to the device, in stream order; the host memory may be reused at once.
+int send(llmdot_hip_ctx* ctx, void* dev, const void* host, size_t n) {
+    if (uint8_t* b = bounce_take(ctx, n)) {
+        memcpy(b, host, n);
+        HIPCHK(launch_copy_bytes(dev, b, n, ctx->stream));
+    } else {
+        HIPCHK(hipMemcpyAsync(dev, host, n, hipMemcpyHostToDevice, ctx->stream));
+    }
     return 0;
 }
 
@@ -275,6 +304,10 @@ extern "C" int32_t llmdot_hip_create(int32_t device, llmdot_hip_ctx** out) {
         return fail(LLMDOT_E_DEVICE, std::string("stream creation failed: ") + hipGetErrorString(e));
     }
     scratch_setup(device);   // llmdot_hip_sample_noalloc reports a failure here
+    if (hipHostMalloc((void**)&ctx->bounce, BOUNCE_BYTES, hipHostMallocDefault) != hipSuccess) {
+        ctx->bounce = nullptr;   // calls copy through the runtime then
+        (void)hipGetLastError();
+    }
     *out = ctx;
     return 0;
 }
@@ -286,6 +319,7 @@ void ctx_release(llmdot_hip_ctx* ctx) {
     for (auto& kv : ctx->weights) (void)hipFree(kv.second.dev);
     for (auto& b : ctx->scratch) b.release();
     for (auto& b : ctx->planes) b.release();
+    if (ctx->bounce) (void)hipHostFree(ctx->bounce);
     if (ctx->am_ints) (void)hipFree(ctx->am_ints);
     if (ctx->am_val) (void)hipFree(ctx->am_val);
     if (ctx->am_idx) (void)hipFree(ctx->am_idx);
@@ -371,8 +405,7 @@ template <typename T>
 int stage_in(llmdot_hip_ctx* ctx, int slot, const T* host, size_t n, T** dev) {
     HIPCHK(ctx->scratch[slot].ensure(sizeof(T) * (n ? n : 1)));
     *dev = reinterpret_cast<T*>(ctx->scratch[slot].p);
-    if (n && host) HIPCHK(hipMemcpyAsync(*dev, host, sizeof(T) * n, hipMemcpyHostToDevice, ctx->stream));
-    return 0;
+    return n && host ? send(ctx, *dev, host, sizeof(T) * n) : 0;
 }
 
 // Activation-plane buffers for M rows of K elements.
@@ -390,8 +423,12 @@ int ctx_planes(llmdot_hip_ctx* ctx, int M, int K, PfPlanes* pl) {
 }
 
 int copy_out(llmdot_hip_ctx* ctx, void* host, const void* dev, size_t nbytes) {
-    HIPCHK(hipMemcpyAsync(host, dev, nbytes, hipMemcpyDeviceToHost, ctx->stream));
+    uint8_t* b = nbytes ? bounce_take(ctx, nbytes) : nullptr;
+    if (b) HIPCHK(launch_copy_bytes(b, dev, nbytes, ctx->stream));
+    else HIPCHK(hipMemcpyAsync(host, dev, nbytes, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
+    if (b) memcpy(host, b, nbytes);
+    ctx->bounce_used = 0;
     return 0;
 }
 
@@ -673,18 +710,42 @@ extern "C" int32_t llmdot_hip_sample(llmdot_hip_ctx* ctx, const float* logits, i
         return fail(LLMDOT_E_UNSUPPORTED, "TopK between " + std::to_string(SAMPLE_MAX_K) + " and the vocabulary size is not supported");
     if (int rc = ensure_device(ctx)) return rc;
     if (int rc = ensure_argmax(ctx, 1)) return rc;
-    float *dl, *dr;
-    int32_t* dh;
-    if (int rc = stage_in(ctx, 0, logits, (size_t)n, &dl)) return rc;
     HIPCHK(ctx->scratch[1].ensure(sizeof(float) * sample_work_floats(n)));
-    if (int rc = stage_in(ctx, 2, recent, (size_t)n_recent, &dh)) return rc;
-    if (int rc = stage_in(ctx, 3, &r, 1, &dr)) return rc;
-    HIPCHK(launch_set_scalar(ctx->am_ints + 1, 1, ctx->stream));   // draw 0
+    // logits, recent tokens, the uniform draw and the draw counter (draw 0), in
+    // one copy where they fit the bounce memory
+    const size_t bytes = sizeof(float) * ((size_t)n + (size_t)n_recent + 2);
+    HIPCHK(ctx->scratch[0].ensure(bytes));
+    float* dl = (float*)ctx->scratch[0].p;
+    int32_t* dh = (int32_t*)(dl + n);
+    float* dr = dl + n + n_recent;
+    int32_t* dstep = (int32_t*)dr + 1;
+    if (uint8_t* b = bounce_take(ctx, bytes)) {
+        const int32_t one = 1;
+        memcpy(b, logits, sizeof(float) * (size_t)n);
+        if (n_recent) memcpy(b + sizeof(float) * (size_t)n, recent, sizeof(int32_t) * (size_t)n_recent);
+        memcpy(b + bytes - 8, &r, 4);
+        memcpy(b + bytes - 4, &one, 4);
+        HIPCHK(launch_copy_bytes(dl, b, bytes, ctx->stream));
+    } else {
+        HIPCHK(hipMemcpyAsync(dl, logits, sizeof(float) * (size_t)n, hipMemcpyHostToDevice, ctx->stream));
+        if (n_recent)
+            HIPCHK(hipMemcpyAsync(dh, recent, sizeof(int32_t) * (size_t)n_recent, hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(hipMemcpyAsync(dr, &r, sizeof(float), hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(launch_set_scalar(dstep, 1, ctx->stream));
+    }
     SampleArgs sa{};
     sa.logits = dl; sa.n = n; sa.inv_temp = 1.0f / opt->temperature;
     sa.top_k = opt->top_k; sa.top_p = opt->top_p; sa.penalty = opt->repeat_penalty; sa.window = opt->repeat_window;
-    sa.hist = dh; sa.hist_base = n_recent; sa.step = ctx->am_ints + 1; sa.rvals = dr;
+    sa.hist = dh; sa.hist_base = n_recent; sa.step = dstep; sa.rvals = dr;
     sa.work = (float*)ctx->scratch[1].p; sa.token_out = ctx->am_ints;
+    // the sampler stores one token: straight to host memory
+    if (uint8_t* b = bounce_take(ctx, sizeof(int32_t))) {
+        sa.token_out = reinterpret_cast<int32_t*>(b);
+        HIPCHK(launch_sample(sa, ctx->stream));
+        HIPCHK(hipStreamSynchronize(ctx->stream));
+        memcpy(token, b, sizeof(int32_t));
+        return 0;
+    }
     HIPCHK(launch_sample(sa, ctx->stream));
     return copy_out(ctx, token, ctx->am_ints, sizeof(int32_t));
 }
@@ -752,7 +813,9 @@ extern "C" int32_t llmdot_hip_memcpy_h2d(llmdot_hip_ctx* ctx, void* dst, const v
 }
 extern "C" int32_t llmdot_hip_memcpy_d2h(llmdot_hip_ctx* ctx, void* dst, const void* src, size_t nbytes) {
     if (!ctx || !dst || !src) return fail(LLMDOT_E_INVALID, "null argument");
-    return copy_out(ctx, dst, src, nbytes);
+    HIPCHK(hipMemcpyAsync(dst, src, nbytes, hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    return 0;
 }
 extern "C" int32_t llmdot_hip_synchronize(llmdot_hip_ctx* ctx) {
     if (!ctx) return fail(LLMDOT_E_INVALID, "null ctx");
@@ -1271,7 +1334,7 @@ int prefill_batched(llmdot_hip_model* m, const int32_t* tokens, int n, int pos0,
     int T = 0;
     for (int c0 = 0; c0 < n; c0 += m->pf_cap) {
         T = std::min(m->pf_cap, n - c0);
-        HIPCHK(hipMemcpyAsync(m->pf_tokens, tokens + c0, sizeof(int32_t) * (size_t)T, hipMemcpyHostToDevice, s));
+        if (int rc = send(m->ctx, m->pf_tokens, tokens + c0, sizeof(int32_t) * (size_t)T)) return rc;
         if (int rc = enqueue_prefill_chunk(m, T, pos0 + c0)) return rc;
     }
     const float* h_last = m->pf_h + (size_t)(T - 1) * m->d.hidden;
@@ -1517,24 +1580,38 @@ int check_pos(llmdot_hip_model* m, int32_t pos) {
 // Device waits that gave up (the attention's chunk-maximum exchange; in the
 // XCD-local form also a chunk placed on another XCD than its kv head's) leave
 // a flag; it is reported once and cleared.
+int report_device_flags(llmdot_hip_model* m, int32_t err) {
+    if (!err) return 0;
+    hipStream_t s = m->ctx->stream;
+    HIPCHK(launch_set_scalar(m_err(m), 0, s));
+    HIPCHK(hipStreamSynchronize(s));
+    return fail(LLMDOT_E_DEVICE, "decode attention: a workgroup gave up waiting for the chunk maxima of its kv "
+                                 "head (spin limit, or with the XCD-local form a chunk on another XCD: "
+                                 "LLMDOT_HIP_ATTN_XCD=0 avoids it); the step's results are invalid");
+}
 int check_device_flags(llmdot_hip_model* m) {
     hipStream_t s = m->ctx->stream;
     int32_t err = 0;
     HIPCHK(hipMemcpyAsync(&err, m_err(m), sizeof(int32_t), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
-    if (err) {
-        HIPCHK(launch_set_scalar(m_err(m), 0, s));
-        HIPCHK(hipStreamSynchronize(s));
-        return fail(LLMDOT_E_DEVICE, "decode attention: a workgroup gave up waiting for the chunk maxima of its kv "
-                                     "head (spin limit, or with the XCD-local form a chunk on another XCD: "
-                                     "LLMDOT_HIP_ATTN_XCD=0 avoids it); the step's results are invalid");
-    }
-    return 0;
+    return report_device_flags(m, err);
 }
 
+// The last step's logits and argmax: one kernel writes them and the device's
+// flags into the bounce memory, and one wait covers all three.
 int fetch_outputs(llmdot_hip_model* m, float* logits, int32_t* am) {
     hipStream_t s = m->ctx->stream;
-    if (logits) HIPCHK(hipMemcpyAsync(logits, m->logits, sizeof(float) * (size_t)m->d.vocab, hipMemcpyDeviceToHost, s));
+    const size_t nl = logits ? sizeof(float) * (size_t)m->d.vocab : 0;
+    if (uint8_t* b = bounce_take(m->ctx, 32 + nl)) {
+        HIPCHK(launch_publish_step(b, m->ints, logits ? m->logits : nullptr, m->d.vocab, s));
+        HIPCHK(hipStreamSynchronize(s));
+        int32_t ints[5];
+        memcpy(ints, b, sizeof ints);
+        if (nl) memcpy(logits, b + 32, nl);
+        if (am) *am = ints[0];
+        return report_device_flags(m, ints[4]);
+    }
+    if (logits) HIPCHK(hipMemcpyAsync(logits, m->logits, nl, hipMemcpyDeviceToHost, s));
     if (am) HIPCHK(hipMemcpyAsync(am, m_token(m), sizeof(int32_t), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     return check_device_flags(m);
@@ -1546,8 +1623,8 @@ extern "C" int32_t llmdot_hip_decode_step(llmdot_hip_model* m, int32_t token, in
     m->gen.active = false;   // the step changes the state a streaming Generate continues from
     if (int rc = check_token(m, token)) return rc;
     if (int rc = check_pos(m, position)) return rc;
-    if (int rc = set_int(m, m_token(m), token)) return rc;
-    if (int rc = set_int(m, m_pos(m), position)) return rc;
+    m->ctx->bounce_used = 0;
+    HIPCHK(launch_set_scalars(m_token(m), token, position, m->ctx->stream));   // token and position
     if (int rc = run_step(m)) return rc;
     return fetch_outputs(m, logits, am);
 }
@@ -1561,6 +1638,7 @@ extern "C" int32_t llmdot_hip_prefill(llmdot_hip_model* m, const int32_t* tokens
     if (int rc = check_pos(m, pos0 + n - 1)) return rc;
     for (int i = 0; i < n; i++)
         if (int rc = check_token(m, tokens[i])) return rc;
+    m->ctx->bounce_used = 0;
     if (use_batched_prefill(m, n)) {
         if (int rc = prefill_batched(m, tokens, n, pos0, false)) return rc;
         return fetch_outputs(m, logits, am);

@@ -101,6 +101,11 @@ hipError_t launch_argmax_finish(const ArgmaxState& st, int ncand, hipStream_t s)
 hipError_t launch_stream_probe(void* buf, size_t nbytes, int mode, uint32_t* sink, hipStream_t s);
 // Position bookkeeping for a captured decode step.
 hipError_t launch_set_scalar(int32_t* dst, int32_t v, hipStream_t s);
+hipError_t launch_set_scalars(int32_t* dst, int32_t v0, int32_t v1, hipStream_t s);   // dst[0], dst[1]
+// nbytes (> 0) between device memory and pinned host memory.
+hipError_t launch_copy_bytes(void* dst, const void* src, size_t nbytes, hipStream_t s);
+// Pinned dst (16-byte aligned): ints[0..4], then, with logits, the n logits from byte 32 on.
+hipError_t launch_publish_step(void* dst, const int32_t* ints, const float* logits, int n, hipStream_t s);
 // Seeded KV contents at positions [0, n) of one cache (kind 0 = K, 1 = V); the values
 // depend only on (seed, layer, kind, position, element).
 hipError_t launch_kv_fill(uint8_t* cache, int kind, int layers, int kv_heads, int context, int hd, int n,

@@ -271,6 +271,37 @@ __global__ __launch_bounds__(WG_BIG) void argmax_finish_kernel(ArgmaxState st, i
 }
 
 __global__ void set_scalar_kernel(int32_t* dst, int32_t v) { *dst = v; }
+__global__ void set_scalars_kernel(int32_t* dst, int32_t v0, int32_t v1) {
+    dst[0] = v0;
+    dst[1] = v1;
+}
+
+// nbytes from src to dst, one of them pinned host memory: bound by the host
+// link, so one 16-byte access per thread, all in flight at once.
+__global__ __launch_bounds__(256) void copy_bytes_kernel(uint8_t* dst, const uint8_t* src, int64_t nbytes, int wide) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (!wide) {
+        if (i < nbytes) dst[i] = src[i];
+        return;
+    }
+    if (16 * i + 16 <= nbytes) {
+        reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+    } else {
+        for (int64_t j = 16 * i; j < nbytes; j++) dst[j] = src[j];
+    }
+}
+// A decode step's state words ints[0..4], and its logits 32 bytes behind them.
+__global__ __launch_bounds__(256) void publish_step_kernel(uint8_t* dst, const int32_t* ints, const float* logits, int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (blockIdx.x == 0 && threadIdx.x < 5) reinterpret_cast<int32_t*>(dst)[threadIdx.x] = ints[threadIdx.x];
+    if (!logits) return;
+    float* out = reinterpret_cast<float*>(dst + 32);
+    if (4 * i + 4 <= n) {
+        reinterpret_cast<float4*>(out)[i] = reinterpret_cast<const float4*>(logits)[i];
+    } else {
+        for (int j = 4 * i; j < n; j++) out[j] = logits[j];
+    }
+}
 
 // Streaming probes: one 16-byte load (or store) per thread.
 __global__ __launch_bounds__(WG) void stream_read_kernel(const uint4* __restrict__ p, size_t n, uint32_t* sink) {
@@ -403,6 +434,22 @@ hipError_t launch_stream_probe(void* buf, size_t nbytes, int mode, uint32_t* sin
     const unsigned grid = (unsigned)((n + WG - 1) / WG);
     if (mode == 0) stream_read_kernel<<<grid, WG, 0, s>>>(reinterpret_cast<const uint4*>(buf), n, sink);
     else stream_write_kernel<<<grid, WG, 0, s>>>(reinterpret_cast<uint4*>(buf), n);
+    return hipGetLastError();
+}
+hipError_t launch_set_scalars(int32_t* dst, int32_t v0, int32_t v1, hipStream_t s) {
+    set_scalars_kernel<<<1, 1, 0, s>>>(dst, v0, v1);
+    return hipGetLastError();
+}
+hipError_t launch_copy_bytes(void* dst, const void* src, size_t nbytes, hipStream_t s) {
+    const bool wide = ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) & 15) == 0;
+    const size_t items = wide ? (nbytes + 15) / 16 : nbytes;
+    copy_bytes_kernel<<<(unsigned)((items + 255) / 256), 256, 0, s>>>((uint8_t*)dst, (const uint8_t*)src,
+                                                                      (int64_t)nbytes, wide);
+    return hipGetLastError();
+}
+hipError_t launch_publish_step(void* dst, const int32_t* ints, const float* logits, int n, hipStream_t s) {
+    const int items = logits ? (n + 3) / 4 : 1;
+    publish_step_kernel<<<(items + 255) / 256, 256, 0, s>>>((uint8_t*)dst, ints, logits, n);
     return hipGetLastError();
 }
 hipError_t launch_set_scalar(int32_t* dst, int32_t v, hipStream_t s) {
