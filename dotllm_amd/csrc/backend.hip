@@ -1296,8 +1296,14 @@ int enqueue_prefill_chunk(llmdot_hip_model* m, int T, int pos0) {
         aa.q_norm = w.q_norm_f; aa.k_norm = w.k_norm_f; aa.eps = d.eps;
         aa.window = d.sliding_window;
         HIPCHK(launch_prefill_rope_kv(aa, s));
+        // the projections' parts are summed: their buffers take the splits'
+        aa.splits = prefill_attn_splits(T, pos0, d.heads, d.kv_fp16, d.sliding_window);
+        aa.part_out = m->pf_parts_q; aa.part_z = m->pf_parts_k; aa.part_max = m->pf_parts_v;
+        aa.part_stride = (int64_t)T * qdim;
+        if (aa.splits * aa.part_stride > PF_PARTS_MAX) aa.splits = 1;
         HIPCHK(launch_prefill_attention(aa, s));
-        HIPCHK(launch_prefill_planes(m->pf_attn, T, qdim, nullptr, 0.f, pl, s));
+        if (aa.splits > 1) HIPCHK(launch_prefill_planes_attn(aa, pl, s));
+        else HIPCHK(launch_prefill_planes(m->pf_attn, T, qdim, nullptr, 0.f, pl, s));
         HIPCHK(proj_add(w.o, qdim));
         HIPCHK(norm_planes(w.ffn_norm_f));
         PfPlan pg{128, 1};   // one launch of gate and up tiles

@@ -240,7 +240,15 @@ struct PfAttnArgs {
     const float *q_norm, *k_norm;
     float eps;
     int window;
+    // keys over `splits` workgroups (prefill_attn_splits; 0 or 1: not): each
+    // split's maxima [splits][heads][T], sums of e V [splits] of [T][heads *
+    // head_dim], part_stride apart, and of e [splits][T][heads]; `out` is not
+    // written then
+    int splits;
+    float *part_max, *part_out, *part_z;
+    int64_t part_stride;
 };
+int prefill_attn_splits(int T, int pos0, int heads, int kv_fp16, int window);
 bool prefill_gemm_supported(uint32_t type, int cols);
 // Optional RmsNorm (norm_w non-null) of each row of x (K <= 16384), then its planes.
 hipError_t launch_prefill_planes(const float* x, int M, int K, const float* norm_w, float eps, const PfPlanes& p,
@@ -251,6 +259,8 @@ hipError_t launch_prefill_planes_add(float* h, const float* parts, int nparts, i
                                      const float* norm_w, float eps, const PfPlanes& p, hipStream_t s);
 hipError_t launch_prefill_planes_swiglu(const float* gate, const float* up, int nparts, int64_t stride, int M, int K,
                                         const PfPlanes& p, hipStream_t s);
+// The same of attention outputs in splits (PfAttnArgs): sum of parts / sum of z.
+hipError_t launch_prefill_planes_attn(const PfAttnArgs& at, const PfPlanes& p, hipStream_t s);
 // One weight matrix of a prefill GEMM: [rows][K] blocks, its output [M][ld]
 // (K part p at out + p * part_stride).
 struct PfMat {

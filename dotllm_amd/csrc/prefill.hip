@@ -110,19 +110,20 @@ struct FVec {
 };
 
 // What a row's planes are made of: the row itself, the row plus the K parts of
-// a projection (the residual add; written back), or SiLU(gate) * up of two
-// projections' K parts.
-enum PfSrc : int { SRC_ROW = 0, SRC_ADD = 1, SRC_SWIGLU = 2 };
+// a projection (the residual add; written back), SiLU(gate) * up of two
+// projections' K parts, or the splits of an attention output over their sums.
+enum PfSrc : int { SRC_ROW = 0, SRC_ADD = 1, SRC_SWIGLU = 2, SRC_ATTN = 3 };
 
 struct PfPlanesArgs {
     float* x;              // SRC_ROW, SRC_ADD: [M][K]
-    const float *pa, *pb;  // SRC_ADD: parts; SRC_SWIGLU: gate and up parts
+    const float *pa, *pb;  // SRC_ADD: parts; SRC_SWIGLU: gate and up parts; SRC_ATTN: sums of e V, of e
     int nparts;
     int64_t stride;
     int K;
     const float* w;        // RmsNorm weights (null: none)
     float eps;
     PfPlanes p;
+    int heads, M;          // SRC_ATTN
 };
 
 // One workgroup of T threads per token row: optional RmsNorm (VectorMath.RmsNorm,
@@ -156,6 +157,13 @@ __global__ __launch_bounds__(T) void pf_planes_kernel(PfPlanesArgs a) {
                 v.load(a.x + at);
                 v.add(y);
                 v.store(a.x + at);
+            } else if constexpr (SRC == SRC_ATTN) {
+                FVec<1> z;   // 4 elements are of one head (head_dim 64, 96 or 128)
+                z.load_parts(a.pb + (int64_t)t * a.heads + base / (K / a.heads), a.nparts, (int64_t)a.M * a.heads);
+                v.load_parts(a.pa + at, a.nparts, a.stride);
+                const float inv = 1.0f / z.v[0];
+#pragma unroll
+                for (int j = 0; j < 4; j++) v.v[j] *= inv;
             } else {
                 FVec<4> g, u;
                 g.load_parts(a.pa + at, a.nparts, a.stride);
@@ -1284,6 +1292,13 @@ hipError_t launch_prefill_planes_swiglu(const float* gate, const float* up, int 
     return launch_planes<false, SRC_SWIGLU>(PfPlanesArgs{nullptr, gate, up, nparts, stride, K, nullptr, 0.f, p}, M, s);
 }
 
+hipError_t launch_prefill_planes_attn(const PfAttnArgs& at, const PfPlanes& p, hipStream_t s) {
+    if (at.splits < 1 || at.part_stride % 4) return hipErrorInvalidValue;
+    return launch_planes<false, SRC_ATTN>(PfPlanesArgs{nullptr, at.part_out, at.part_z, at.splits, at.part_stride,
+                                                       at.heads * at.head_dim, nullptr, 0.f, p, at.heads, at.T},
+                                          at.T, s);
+}
+
 namespace {
 hipError_t launch_gemm_type(uint32_t type, int epi, const PfGemmArgs& a, int tm, hipStream_t s) {
     switch (type) {
@@ -1419,7 +1434,7 @@ hipError_t launch_prefill_attention(const PfAttnArgs& a, hipStream_t s) {
     // 128 behind 3900: 276 / 88; 256 workgroups of 512 keys 35 / 19, of 2048
     // keys 119 / 58; 416 of 777: 60 / 36).
     const int wgs = (a.T + AQ - 1) / AQ * a.heads;
-    if (!a.kv_fp16 || wgs < 256 || (wgs < 512 && a.pos0 + a.T <= 2048)) return launch_prefill_attn_wave(a, s);
+    if (a.splits > 1 || !a.kv_fp16 || wgs < 256 || (wgs < 512 && a.pos0 + a.T <= 2048)) return launch_prefill_attn_wave(a, s);
     switch (a.head_dim) {
     case 64: return launch_attn_hd<64>(a, s);
     case 96: return launch_attn_hd<96>(a, s);

@@ -31,6 +31,8 @@
 #include "common.h"
 #include "kernels.h"
 
+#include <algorithm>
+
 namespace llmdot {
 
 namespace {
@@ -176,7 +178,13 @@ struct Attn {
     }
 };
 
-template <int HD, bool F16, int W>
+// MODE: all of it, or with the keys also spread over blockIdx.y of a.splits
+// workgroups, the maxima (to a.part_max) and then the sums (to a.part_out and
+// a.part_z, added up where they are read) as a launch each: a CU reads rows at
+// about 50 GB/s, so with few query blocks only more CUs shorten it.
+enum AttnMode { ATTN_ALL = 0, ATTN_MAX = 1, ATTN_SUM = 2 };
+
+template <int HD, bool F16, int W, int MODE>
 __global__ __launch_bounds__(64 * W) void pf_attn_wave_kernel(PfAttnArgs a) {
     using A = Attn<HD, F16>;
     constexpr int DPL = A::DPL, NC = A::NC, KT = A::KT, KSTEP = A::KSTEP, NT = HD / 16;
@@ -201,16 +209,18 @@ __global__ __launch_bounds__(64 * W) void pf_attn_wave_kernel(PfAttnArgs a) {
     const int n8 = first + ((a.pos0 + tqc + 1 - first) & ~7);
     const int nkeys = a.pos0 + min(t0 + QB, a.T);
     const int64_t base = (int64_t)kvh * a.context * HD;
-    const int j_first = jstart + wv * KSTEP;
+    const int split = MODE == ATTN_ALL ? 0 : (int)blockIdx.y;
+    const int j_step = (MODE == ATTN_ALL ? W : W * a.splits) * KSTEP;
+    const int j_first = jstart + (split * W + wv) * KSTEP;
 
     // pass 1: the queries' maxima over this wavefront's keys
     float m = -INFINITY;
-    {
+    if constexpr (MODE != ATTN_SUM) {
         typename A::KFrag cur, nxt;
         A::load_k(nxt, a.kcache, base, j_first, nkeys, lr, lk);
-        for (int j0 = j_first; j0 < nkeys; j0 += W * KSTEP) {
+        for (int j0 = j_first; j0 < nkeys; j0 += j_step) {
             cur = nxt;
-            A::load_k(nxt, a.kcache, base, j0 + W * KSTEP, nkeys, lr, lk);
+            A::load_k(nxt, a.kcache, base, j0 + j_step, nkeys, lr, lk);
 #pragma unroll
             for (int kt = 0; kt < KT; kt++) {
                 const f4 c = at.scores(cur, kt);
@@ -222,13 +232,23 @@ __global__ __launch_bounds__(64 * W) void pf_attn_wave_kernel(PfAttnArgs a) {
             }
         }
     }
-    m = fmaxf(m, fx(lane_xor16, m));
-    m = fmaxf(m, fx(lane_xor32, m));
-    if (lk == 0) mx[wv][lr] = m;
-    __syncthreads();
-    float mq = mx[0][lr];
+    float mq;
+    if constexpr (MODE != ATTN_SUM) {
+        m = fmaxf(m, fx(lane_xor16, m));
+        m = fmaxf(m, fx(lane_xor32, m));
+        if (lk == 0) mx[wv][lr] = m;
+        __syncthreads();
+        mq = mx[0][lr];
 #pragma unroll
-    for (int w = 1; w < W; w++) mq = fmaxf(mq, mx[w][lr]);
+        for (int w = 1; w < W; w++) mq = fmaxf(mq, mx[w][lr]);
+        if constexpr (MODE == ATTN_MAX) {
+            if (tid < QB && tq < a.T) a.part_max[((int64_t)split * a.heads + h) * a.T + tq] = mq;
+            return;
+        }
+    } else {
+        mq = -INFINITY;
+        for (int i = 0; i < a.splits; i++) mq = fmaxf(mq, a.part_max[((int64_t)i * a.heads + h) * a.T + tqc]);
+    }
 
     // pass 2: the same scores, softmax numerators (ExpApprox on the vector
     // lanes, expf on the tail, VM:215-258), their sum and e . V
@@ -243,11 +263,11 @@ __global__ __launch_bounds__(64 * W) void pf_attn_wave_kernel(PfAttnArgs a) {
     typename A::VFrag vn, vf;
     A::load_k(kn, a.kcache, base, j_first, nkeys, lr, lk);
     A::load_v(vn, a.vcache, base, j_first, nkeys, lr, lk);
-    for (int j0 = j_first; j0 < nkeys; j0 += W * KSTEP) {
+    for (int j0 = j_first; j0 < nkeys; j0 += j_step) {
         kf = kn;
         vf = vn;
-        A::load_k(kn, a.kcache, base, j0 + W * KSTEP, nkeys, lr, lk);
-        A::load_v(vn, a.vcache, base, j0 + W * KSTEP, nkeys, lr, lk);
+        A::load_k(kn, a.kcache, base, j0 + j_step, nkeys, lr, lk);
+        A::load_v(vn, a.vcache, base, j0 + j_step, nkeys, lr, lk);
         float ev[KT][4];
 #pragma unroll
         for (int kt = 0; kt < KT; kt++) {
@@ -331,10 +351,12 @@ __global__ __launch_bounds__(64 * W) void pf_attn_wave_kernel(PfAttnArgs a) {
         const float zq = __shfl(z, ql, 64);
         const int t = t0 + ql;
         if (t < a.T) {
-            const float inv = 1.0f / zq;
+            const float inv = MODE == ATTN_SUM ? 1.0f : 1.0f / zq;
+            float* const out = MODE == ATTN_SUM ? a.part_out + split * a.part_stride : a.out;
+            if (MODE == ATTN_SUM && lr == 0) a.part_z[((int64_t)split * a.T + t) * a.heads + h] = zq;
 #pragma unroll
             for (int c = 0; c < NC; c++) {
-                float* o = a.out + (int64_t)t * (a.heads * HD) + h * HD + 16 * DPL * c + DPL * lr;
+                float* o = out + (int64_t)t * (a.heads * HD) + h * HD + 16 * DPL * c + DPL * lr;
 #pragma unroll
                 for (int j = 0; j < DPL; j++) o[j] = (F16 ? acc[c][j][r] * (1.0f / P14) : acc[c][j][r]) * inv;
             }
@@ -348,14 +370,36 @@ hipError_t launch_wave(const PfAttnArgs& a, hipStream_t s) {
     // 8 wavefronts a workgroup where there is one workgroup a CU at most (128
     // tokens behind 3900: 88 us against 103 with 4), else 4 (256 tokens, 512
     // workgroups: 16 against 20)
-    if (grid <= 256) pf_attn_wave_kernel<HD, F16, 8><<<grid, 512, 0, s>>>(a);
-    else pf_attn_wave_kernel<HD, F16, 4><<<grid, 256, 0, s>>>(a);
+    if (a.splits > 1) {
+        pf_attn_wave_kernel<HD, F16, 8, ATTN_MAX><<<dim3(grid, a.splits), 512, 0, s>>>(a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        pf_attn_wave_kernel<HD, F16, 8, ATTN_SUM><<<dim3(grid, a.splits), 512, 0, s>>>(a);
+    } else if (grid <= 256) {
+        pf_attn_wave_kernel<HD, F16, 8, ATTN_ALL><<<grid, 512, 0, s>>>(a);
+    } else {
+        pf_attn_wave_kernel<HD, F16, 4, ATTN_ALL><<<grid, 256, 0, s>>>(a);
+    }
     return hipGetLastError();
 }
 
 }  // namespace
 
+int prefill_attn_splits(int T, int pos0, int heads, int kv_fp16, int window) {
+    const int wgs = (T + QB - 1) / QB * heads;
+    // where at least half of the CUs have no workgroup: 64 workgroups of 1823 keys
+    // (23 tokens, 32 heads of 128) 42 us, in 4 splits 10 + 15; with a workgroup
+    // on every CU the row loads are already spread
+    if (wgs > 128) return 1;
+    // steps of 32 (16) keys per wavefront; two are left to each
+    const int keys = window > 0 ? std::min(pos0 + T, window + QB) : pos0 + T, step = kv_fp16 ? 32 : 16;
+    const int per_wave = (keys + 8 * step - 1) / (8 * step);
+    return std::max(1, std::min({16, 256 / wgs, per_wave / 2}));
+}
+
 hipError_t launch_prefill_attn_wave(const PfAttnArgs& a, hipStream_t s) {
+    if (a.splits > 1 && (!a.part_max || !a.part_out || !a.part_z || a.part_stride < (int64_t)a.T * a.heads * a.head_dim))
+        return hipErrorInvalidValue;
     switch (a.head_dim) {
     case 64: return a.kv_fp16 ? launch_wave<64, true>(a, s) : launch_wave<64, false>(a, s);
     case 96: return a.kv_fp16 ? launch_wave<96, true>(a, s) : launch_wave<96, false>(a, s);

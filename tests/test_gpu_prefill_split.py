@@ -57,3 +57,20 @@ def test_batched_matmul_tiles_and_parts(hip, t, k, m, n):
     y = np.zeros(m * n, dtype=np.float32)
     hip.mat_mul(a.reshape(-1), w, y, t, k, n)
     assert row_rel_err(y.reshape(m, n), ref) <= FP32_LEVEL
+
+
+@pytest.mark.parametrize("model,n,split,kv_fp16", [("tiny", 1030, 1029, True), ("tiny", 1030, 1020, False),
+                                                   ("phi3mini", 560, 545, True), ("small5", 1100, 1093, False),
+                                                   ("small5", 1100, 1080, True)])
+def test_prefill_attention_splits(hip, oracle_threads, model, n, split, kv_fp16):  # noqa: F811
+    """A few queries behind many keys: the keys over 2 to 8 workgroups as well,
+    some splits without keys for a wavefront."""
+    spec = dict(synth.SPECS[model], layers=1)
+    img = synth.build_image(model, seed=1234, spec=spec, context=1120)
+    _prompt_check(hip, img, synth.prompt(32000, n, seed=7), 1120, kv_fp16, [0], split=split)
+
+
+def test_prefill_attention_splits_window(hip):
+    """The same with a window: splits start at its first key."""
+    img = synth.build_image("tiny", seed=1234, context=1120, sliding_window=700)
+    _prompt_check(hip, img, synth.prompt(32000, 1000, seed=7), 1120, True, [0, 3], split=985)
