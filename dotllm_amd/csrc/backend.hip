@@ -106,6 +106,9 @@ struct llmdot_hip_ctx {
     // (BOUNCE_BYTES; null: not available): copied by the host on one side, by a
     // kernel on the stream on the other.  Every pageable copy of the runtime is
     // a wait of its own, 10-20 us however small; a decode step made three.
+    // Bytes handed out belong to queued kernels until the stream has been waited
+    // for, which can be calls later (llmdot_hip_generate_begin returns with its
+    // prompt still queued): only wait_stream gives them back.
     uint8_t* bounce = nullptr;
     size_t bounce_used = 0;
     hipEvent_t fork = nullptr, join[2] = {nullptr, nullptr};
@@ -126,16 +129,24 @@ struct llmdot_hip_ctx {
 
 namespace {
 
-// Starts a call: its device, and all of the bounce memory.
 int ensure_device(llmdot_hip_ctx* ctx) {
     HIPCHK(hipSetDevice(ctx->device));
+    return 0;
+}
+
+// Waits for everything on the stream: no queued kernel reads or writes the
+// bounce memory any more, so all of it is free again (a result the caller still
+// has to copy out of it stays there until the next bounce_take).
+int wait_stream(llmdot_hip_ctx* ctx) {
+    HIPCHK(hipStreamSynchronize(ctx->stream));
     ctx->bounce_used = 0;
     return 0;
 }
 
 constexpr size_t BOUNCE_BYTES = 1 << 20;
 
-// n bytes of the bounce memory for the rest of this call; null if they do not fit.
+// n bytes of the bounce memory until the next wait_stream; null if they do not
+// fit beside those in use (the caller then copies through the runtime).
 uint8_t* bounce_take(llmdot_hip_ctx* ctx, size_t n) {
     if (!ctx->bounce || n > BOUNCE_BYTES - ctx->bounce_used) return nullptr;
     uint8_t* p = ctx->bounce + ctx->bounce_used;
@@ -426,9 +437,8 @@ int copy_out(llmdot_hip_ctx* ctx, void* host, const void* dev, size_t nbytes) {
     uint8_t* b = nbytes ? bounce_take(ctx, nbytes) : nullptr;
     if (b) HIPCHK(launch_copy_bytes(b, dev, nbytes, ctx->stream));
     else HIPCHK(hipMemcpyAsync(host, dev, nbytes, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    if (int rc = wait_stream(ctx)) return rc;
     if (b) memcpy(host, b, nbytes);
-    ctx->bounce_used = 0;
     return 0;
 }
 
@@ -531,7 +541,7 @@ int rope_common(llmdot_hip_ctx* ctx, float* q, float* k, int head_dim, const std
     HIPCHK(launch_rope(dq, same ? dq : dk, dc, ds, half, same, ctx->stream));
     HIPCHK(hipMemcpyAsync(q, dq, sizeof(float) * (size_t)head_dim, hipMemcpyDeviceToHost, ctx->stream));
     if (!same) HIPCHK(hipMemcpyAsync(k, dk, sizeof(float) * (size_t)head_dim, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    if (int rc = wait_stream(ctx)) return rc;
     return 0;
 }
 }  // namespace
@@ -742,7 +752,7 @@ extern "C" int32_t llmdot_hip_sample(llmdot_hip_ctx* ctx, const float* logits, i
     if (uint8_t* b = bounce_take(ctx, sizeof(int32_t))) {
         sa.token_out = reinterpret_cast<int32_t*>(b);
         HIPCHK(launch_sample(sa, ctx->stream));
-        HIPCHK(hipStreamSynchronize(ctx->stream));
+        if (int rc = wait_stream(ctx)) return rc;
         memcpy(token, b, sizeof(int32_t));
         return 0;
     }
@@ -808,18 +818,18 @@ extern "C" int32_t llmdot_hip_device_free(llmdot_hip_ctx* ctx, void* dptr) {
 extern "C" int32_t llmdot_hip_memcpy_h2d(llmdot_hip_ctx* ctx, void* dst, const void* src, size_t nbytes) {
     if (!ctx || !dst || !src) return fail(LLMDOT_E_INVALID, "null argument");
     HIPCHK(hipMemcpyAsync(dst, src, nbytes, hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    if (int rc = wait_stream(ctx)) return rc;
     return 0;
 }
 extern "C" int32_t llmdot_hip_memcpy_d2h(llmdot_hip_ctx* ctx, void* dst, const void* src, size_t nbytes) {
     if (!ctx || !dst || !src) return fail(LLMDOT_E_INVALID, "null argument");
     HIPCHK(hipMemcpyAsync(dst, src, nbytes, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    if (int rc = wait_stream(ctx)) return rc;
     return 0;
 }
 extern "C" int32_t llmdot_hip_synchronize(llmdot_hip_ctx* ctx) {
     if (!ctx) return fail(LLMDOT_E_INVALID, "null ctx");
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    if (int rc = wait_stream(ctx)) return rc;
     return 0;
 }
 
@@ -1570,7 +1580,7 @@ extern "C" int32_t llmdot_hip_model_reset(llmdot_hip_model* m) {
     m->gen.active = false;
     if (int rc = set_int(m, m_pos(m), 0)) return rc;
     if (int rc = set_int(m, m_step(m), 0)) return rc;
-    HIPCHK(hipStreamSynchronize(m->ctx->stream));
+    if (int rc = wait_stream(m->ctx)) return rc;
     return 0;
 }
 
@@ -1590,7 +1600,7 @@ int report_device_flags(llmdot_hip_model* m, int32_t err) {
     if (!err) return 0;
     hipStream_t s = m->ctx->stream;
     HIPCHK(launch_set_scalar(m_err(m), 0, s));
-    HIPCHK(hipStreamSynchronize(s));
+    if (int rc = wait_stream(m->ctx)) return rc;
     return fail(LLMDOT_E_DEVICE, "decode attention: a workgroup gave up waiting for the chunk maxima of its kv "
                                  "head (spin limit, or with the XCD-local form a chunk on another XCD: "
                                  "LLMDOT_HIP_ATTN_XCD=0 avoids it); the step's results are invalid");
@@ -1599,7 +1609,7 @@ int check_device_flags(llmdot_hip_model* m) {
     hipStream_t s = m->ctx->stream;
     int32_t err = 0;
     HIPCHK(hipMemcpyAsync(&err, m_err(m), sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
+    if (int rc = wait_stream(m->ctx)) return rc;
     return report_device_flags(m, err);
 }
 
@@ -1610,7 +1620,7 @@ int fetch_outputs(llmdot_hip_model* m, float* logits, int32_t* am) {
     const size_t nl = logits ? sizeof(float) * (size_t)m->d.vocab : 0;
     if (uint8_t* b = bounce_take(m->ctx, 32 + nl)) {
         HIPCHK(launch_publish_step(b, m->ints, logits ? m->logits : nullptr, m->d.vocab, s));
-        HIPCHK(hipStreamSynchronize(s));
+        if (int rc = wait_stream(m->ctx)) return rc;
         int32_t ints[5];
         memcpy(ints, b, sizeof ints);
         if (nl) memcpy(logits, b + 32, nl);
@@ -1619,7 +1629,7 @@ int fetch_outputs(llmdot_hip_model* m, float* logits, int32_t* am) {
     }
     if (logits) HIPCHK(hipMemcpyAsync(logits, m->logits, nl, hipMemcpyDeviceToHost, s));
     if (am) HIPCHK(hipMemcpyAsync(am, m_token(m), sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
+    if (int rc = wait_stream(m->ctx)) return rc;
     return check_device_flags(m);
 }
 }  // namespace
@@ -1629,7 +1639,6 @@ extern "C" int32_t llmdot_hip_decode_step(llmdot_hip_model* m, int32_t token, in
     m->gen.active = false;   // the step changes the state a streaming Generate continues from
     if (int rc = check_token(m, token)) return rc;
     if (int rc = check_pos(m, position)) return rc;
-    m->ctx->bounce_used = 0;
     HIPCHK(launch_set_scalars(m_token(m), token, position, m->ctx->stream));   // token and position
     if (int rc = run_step(m)) return rc;
     return fetch_outputs(m, logits, am);
@@ -1644,7 +1653,6 @@ extern "C" int32_t llmdot_hip_prefill(llmdot_hip_model* m, const int32_t* tokens
     if (int rc = check_pos(m, pos0 + n - 1)) return rc;
     for (int i = 0; i < n; i++)
         if (int rc = check_token(m, tokens[i])) return rc;
-    m->ctx->bounce_used = 0;
     if (use_batched_prefill(m, n)) {
         if (int rc = prefill_batched(m, tokens, n, pos0, false)) return rc;
         return fetch_outputs(m, logits, am);
@@ -1765,7 +1773,7 @@ int generate_next(llmdot_hip_model* m, int32_t max_k, int32_t* tokens_out, int32
                                   hipMemcpyDeviceToHost, s));
     }
     HIPCHK(hipMemcpyAsync(tokens_out, m->token_log + g.yielded, sizeof(int32_t) * (size_t)want, hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
+    if (int rc = wait_stream(m->ctx)) return rc;
     if (int rc = check_device_flags(m)) { g.active = false; return rc; }
     int n = want;
     bool eos_hit = false;
@@ -1828,7 +1836,7 @@ extern "C" int32_t llmdot_hip_kv_read(llmdot_hip_model* m, int32_t layer, int32_
     const auto& d = m->d;
     const size_t elt = d.kv_fp16 ? 2 : 4;
     std::vector<uint8_t> kb((size_t)d.head_dim * elt), vb((size_t)d.head_dim * elt);
-    HIPCHK(hipStreamSynchronize(m->ctx->stream));
+    if (int rc = wait_stream(m->ctx)) return rc;
     for (int h = 0; h < d.kv_heads; h++) {
         const size_t off = (size_t)layer * m->kv_layer_bytes + (((size_t)h * d.context + position) * d.head_dim) * elt;
         HIPCHK(hipMemcpy(kb.data(), m->kcache + off, kb.size(), hipMemcpyDeviceToHost));
@@ -1873,7 +1881,7 @@ extern "C" int32_t llmdot_hip_model_kv_fill_random(llmdot_hip_model* m, int32_t 
     const auto& d = m->d;
     HIPCHK(launch_kv_fill(m->kcache, 0, d.layers, d.kv_heads, d.context, d.head_dim, n, seed, d.kv_fp16, m->ctx->stream));
     HIPCHK(launch_kv_fill(m->vcache, 1, d.layers, d.kv_heads, d.context, d.head_dim, n, seed, d.kv_fp16, m->ctx->stream));
-    HIPCHK(hipStreamSynchronize(m->ctx->stream));
+    if (int rc = wait_stream(m->ctx)) return rc;
     return 0;
 }
 
@@ -1891,7 +1899,7 @@ extern "C" int32_t llmdot_hip_model_time_prefill(llmdot_hip_model* m, const int3
     hipEvent_t e0, e1;
     HIPCHK(hipEventCreate(&e0));
     HIPCHK(hipEventCreate(&e1));
-    HIPCHK(hipStreamSynchronize(s));
+    if (int rc = wait_stream(m->ctx)) return rc;
     HIPCHK(hipEventRecord(e0, s));
     int rc = prefill_batched(m, tokens, n, pos0, false);
     if (rc == 0) {
@@ -1922,7 +1930,7 @@ extern "C" int32_t llmdot_hip_model_time_decode(llmdot_hip_model* m, int32_t fir
     hipGraphExec_t kg = nullptr;
     if (per_kernel) {
         hipGraph_t g = nullptr;
-        HIPCHK(hipStreamSynchronize(s));
+        if (int rc = wait_stream(m->ctx)) return rc;
         HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         hipError_t le = hipSuccess;
         for (int l = 0; l < m->d.layers && le == hipSuccess; l++) le = launch_gate_up(m, l);
@@ -1938,7 +1946,7 @@ extern "C" int32_t llmdot_hip_model_time_decode(llmdot_hip_model* m, int32_t fir
     hipEvent_t e0, e1;
     HIPCHK(hipEventCreate(&e0));
     HIPCHK(hipEventCreate(&e1));
-    HIPCHK(hipStreamSynchronize(s));
+    if (int rc = wait_stream(m->ctx)) return rc;
     HIPCHK(hipEventRecord(e0, s));
     int launches = 0;
     hipError_t re = hipSuccess;

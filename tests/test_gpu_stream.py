@@ -135,3 +135,52 @@ def test_stream_sampled_equals_one_shot(hip, tiny_image):
         assert list(eng.generate(prompt, opts, chunk=24, draws=draws)) == ref
     finally:
         eng.dispose()
+
+
+@pytest.mark.parametrize("between", ["prefill", "add", "sample"])
+def test_stream_prompt_still_queued(hip, tiny_image, monkeypatch, between):
+    """llmdot_hip_generate_begin returns with its prompt queued: calls on the
+    same context before the first _next (another model's prompt of in-range
+    tokens, op-level calls over most of the pinned memory) must leave the token
+    ids that later chunks still have to read as they are.  400 tokens in chunks
+    of 16; the tokens equal the one-shot call's."""
+    monkeypatch.setenv("LLMDOT_HIP_PREFILL_CHUNK", "16")
+    prompt, other = synth.prompt(32000, 400, seed=21), synth.prompt(32000, 400, seed=22)
+    model = LoadedModel.load(tiny_image)
+    eng, eng2 = (InferenceEngine(model, hip, kv_fp16=True, context=448) for _ in range(2))
+    a, y = np.ones(65536, np.float32), np.zeros(65536, np.float32)
+    x = np.random.default_rng(1).normal(0, 2, 200000).astype(np.float32)
+    try:
+        ref, _ = eng.generate_all(prompt, greedy(8))
+        want, _ = eng2.prefill(other, 0)
+        for _ in range(2):
+            assert _begin(eng, prompt, 8) == 0
+            if between == "prefill":
+                assert np.array_equal(eng2.prefill(other, 0)[0], want)
+            elif between == "add":
+                hip.add(a, a, y)
+                assert np.all(y == 2.0)
+            else:
+                assert hip.sample(x, SamplingOptions(top_k=1), [], 0.5) == int(np.argmax(x))
+            rc, toks, _, done = _next(eng, 8)
+            assert rc == 0 and done and toks == ref
+    finally:
+        eng.dispose()
+        eng2.dispose()
+
+
+def test_stream_begun_many_times(hip, tiny_image, monkeypatch):
+    """Prompts begun again and again with nothing that waits in between: more
+    chunks than the pinned memory has room for, so that the last ones pass
+    through the runtime's copies; then the one-shot call's tokens."""
+    monkeypatch.setenv("LLMDOT_HIP_PREFILL_CHUNK", "16")
+    prompt = synth.prompt(32000, 400, seed=23)
+    eng = InferenceEngine(LoadedModel.load(tiny_image), hip, kv_fp16=True, context=448)
+    try:
+        ref, _ = eng.generate_all(prompt, greedy(8))
+        for _ in range(170):   # 25 chunks each, 256 bytes a chunk: 1 MiB is 163 prompts
+            assert _begin(eng, prompt, 8) == 0
+        rc, toks, _, done = _next(eng, 8)
+        assert rc == 0 and done and toks == ref
+    finally:
+        eng.dispose()
