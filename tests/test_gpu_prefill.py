@@ -149,9 +149,10 @@ def _prompt_check(hip, img, prompt, ctx, kv_fp16, layers, split=None):
 
 @pytest.mark.parametrize("kv_fp16", [True, False])
 def test_prefill_tiny_multi_tile(hip, tiny_image, kv_fp16):
-    """tiny Q8_0, MHA head_dim 64: 200 tokens = 2 token tiles, 4 key tiles.
-    Every projection launch has under 128 tiles, so Q, K, V and O run in 8 K
-    parts and down (44 steps) in 4, summed by the next kernel."""
+    """tiny Q8_0, MHA head_dim 64: 200 tokens = 4 token tiles of 64, 4 key tiles
+    (of 64).  Every projection launch leaves CUs idle, so Q + K, V, O and gate
+    and up run in 4 K parts (the 4 units of 512 columns) and down in 11 (of 1408),
+    summed by the next kernel."""
     prompt = synth.prompt(32000, 200, seed=17)
     _prompt_check(hip, tiny_image, prompt, 256, kv_fp16, [0, 3])
 
@@ -218,14 +219,28 @@ def test_prefill_mistral7b(hip, oracle_threads):
 
 
 def test_prefill_64_token_tiles_bit_identical(hip, monkeypatch):
-    """1B shape, 1024-token prompt: Q, O and down have 128 tiles of 128 tokens,
-    which run as 64-token tiles (Q STORE, O and down ADD into the residual),
-    with Q4_K, Q6_K and the min term.  Every output's sum runs in the same
-    order as with 128-token tiles, so the last logits and the KV cache must
-    be bit-identical with the 64-token tiles turned off."""
+    """1B shape, 1024-token prompt: V (Q6_K, 4 K parts) and O (Q4_K with the min
+    term, 2 parts) run as 64-token tiles, storing parts.  Every output's sum
+    runs in the same order as with 128-token tiles, so the last logits and the
+    KV cache must be bit-identical with the 64-token tiles turned off."""
     n, ctx = 1024, 1040
     img = synth.build_image("llama1b", seed=1234, context=ctx)
-    prompt = synth.prompt(128256, n, seed=29)
+    _tiles_64_check(hip, monkeypatch, img, synth.prompt(128256, n, seed=29), ctx, (0, 7, 15), (0, 511, 1023))
+
+
+@pytest.mark.parametrize("model,n", [("tiny", 200), ("small5", 150), ("llama1b", 40), ("phi3mini", 130)])
+def test_prefill_64_token_tiles_add_bit_identical(hip, monkeypatch, model, n):
+    """The same with the K parts turned off, where O and down ADD 64-token tiles
+    into the residual (as they do unforced for wide models, 443 x 9088 x 10752
+    for one): Q8_0, Q5_K, Q4_K and Q6_K."""
+    monkeypatch.setenv("LLMDOT_HIP_PF_NO_SPLIT", "1")
+    spec = dict(synth.SPECS[model], layers=2)
+    img = synth.build_image(model, seed=1234, spec=spec, context=256)
+    _tiles_64_check(hip, monkeypatch, img, synth.prompt(32000, n, seed=29), 256, (0, 1), (0, n // 2, n - 1))
+
+
+def _tiles_64_check(hip, monkeypatch, img, prompt, ctx, layers, positions):
+    """Last logits, argmax and KV rows with and without 64-token tiles, bit for bit."""
     runs = []
     for off in (False, True):
         if off:
@@ -235,7 +250,7 @@ def test_prefill_64_token_tiles_bit_identical(hip, monkeypatch):
         eng = InferenceEngine(LoadedModel.load(img), hip, kv_fp16=True, context=ctx)
         try:
             logits, am = eng.prefill(prompt, 0)
-            kv = [eng.kv_read(layer, pos) for layer in (0, 7, 15) for pos in (0, 511, 1023)]
+            kv = [eng.kv_read(layer, pos) for layer in layers for pos in positions]
         finally:
             eng.dispose()
         runs.append((np.array(logits, copy=True), am, kv))

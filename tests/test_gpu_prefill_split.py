@@ -4,14 +4,35 @@ keys spread over a workgroup's wavefronts, projections in uneven K parts.
 
 Bounds: those of test_gpu_prefill.py (`_prompt_check`).
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from dotllm_amd import Q4_0, Q4_K, Q5_K, Q6_K, Q8_0, synth
+from dotllm_amd import Q4_0, Q4_K, Q5_K, Q6_K, Q8_0, _lib, synth
+from dotllm_amd.engine import InferenceEngine, LoadedModel
 from oracle import oracle as O
-from test_gpu_prefill import FP32_LEVEL, _prompt_check, oracle_threads, random_blocks, row_rel_err  # noqa: F401
+from oracle_pair import KV_MARGIN, OraclePair
+from test_gpu_prefill import (FP32_LEVEL, KV_MIN, _prompt_check, oracle_threads, random_blocks,  # noqa: F401
+                              row_rel_err)
 
 pytestmark = pytest.mark.gpu
+PARTS_MAX = 512 * 128 * 128   # floats of a parts buffer
+
+
+def host_fn(name, args, restype=C.c_int):
+    """One of the library's own launch rules (host code, not part of the C ABI):
+    the tests assert that their sizes take the path they are about."""
+    f = getattr(_lib.lib(), f"_ZN6llmdot{len(name)}{name}E{args}")
+    f.restype = restype
+    f.argtypes = [{"i": C.c_int, "j": C.c_uint32, "l": C.c_int64}[a] for a in args]
+    return f
+
+
+def plan(t, m, n, k):
+    """(tokens per tile, K parts) of a batched product (prefill_plan)."""
+    v = host_fn("prefill_plan", "jiiil", C.c_int64)(t, m, n, k, PARTS_MAX)
+    return v & 0xFFFFFFFF, v >> 32
 
 
 @pytest.mark.parametrize("rot", [60, 24, 2])
@@ -46,10 +67,12 @@ def test_prefill_attention_512_queries_groups(hip, oracle_threads):  # noqa: F81
 
 
 @pytest.mark.parametrize("t,k", [(Q4_K, 2816), (Q5_K, 256), (Q6_K, 1280), (Q8_0, 1408), (Q8_0, 32), (Q4_0, 4192)])
-@pytest.mark.parametrize("m,n", [(2, 129), (32, 300), (33, 96), (64, 2000), (65, 128), (140, 520)])
-def test_batched_matmul_tiles_and_parts(hip, t, k, m, n):
-    """Edges of the 32-, 64- and 128-token tiles; K in uneven parts, one unit
-    only, and a last unit of fewer than 4 blocks."""
+@pytest.mark.parametrize("m,n,tile", [(2, 129, 32), (32, 300, 32), (33, 96, 64), (64, 2000, 64), (65, 128, 64),
+                                      (140, 520, 64), (1030, 140, 128)])
+def test_batched_matmul_tiles_and_parts(hip, t, k, m, n, tile):
+    """Edges of the 32- and 64-token tiles and a ragged last 128-token tile; K in
+    uneven parts, one unit only, and a last unit of fewer than 4 blocks."""
+    assert plan(t, m, n, k)[0] == tile
     rng = np.random.default_rng(m + n + k)
     w = random_blocks(t, n, k, m + n)
     a = rng.normal(0, 1, size=(m, k)).astype(np.float32)
@@ -59,18 +82,44 @@ def test_batched_matmul_tiles_and_parts(hip, t, k, m, n):
     assert row_rel_err(y.reshape(m, n), ref) <= FP32_LEVEL
 
 
-@pytest.mark.parametrize("model,n,split,kv_fp16", [("tiny", 1030, 1029, True), ("tiny", 1030, 1020, False),
-                                                   ("phi3mini", 560, 545, True), ("small5", 1100, 1093, False),
-                                                   ("small5", 1100, 1080, True)])
-def test_prefill_attention_splits(hip, oracle_threads, model, n, split, kv_fp16):  # noqa: F811
-    """A few queries behind many keys: the keys over 2 to 8 workgroups as well,
-    some splits without keys for a wavefront."""
-    spec = dict(synth.SPECS[model], layers=1)
-    img = synth.build_image(model, seed=1234, spec=spec, context=1120)
-    _prompt_check(hip, img, synth.prompt(32000, n, seed=7), 1120, kv_fp16, [0], split=split)
+# heads of 96 at the smallest widths the phi3 mix takes
+SMALL96 = dict(synth.SPECS["phi3mini"], hidden=768, layers=2, heads=8, kv_heads=8, ffn=1024, vocab=4096)
 
 
-def test_prefill_attention_splits_window(hip):
-    """The same with a window: splits start at its first key."""
-    img = synth.build_image("tiny", seed=1234, context=1120, sliding_window=700)
-    _prompt_check(hip, img, synth.prompt(32000, 1000, seed=7), 1120, True, [0, 3], split=985)
+@pytest.mark.parametrize("model,t,pos0,kv_fp16,window,splits", [
+    ("tiny", 16, 1150, True, 0, 2), ("tiny", 10, 1020, False, 0, 4), ("tiny", 40, 2500, True, 0, 5),
+    ("tiny", 5, 8100, True, 0, 16), ("small5", 20, 1080, True, 0, 2), ("small5", 7, 1093, False, 0, 4),
+    ("small5", 15, 4000, True, 0, 8), ("small5", 5, 4090, False, 0, 16), ("small96", 2, 1027, True, 0, 2),
+    ("small96", 15, 3000, False, 0, 12), ("small96", 33, 4063, True, 0, 8),
+    ("tiny", 15, 3000, True, 2100, 4), ("small5", 20, 4070, True, 1500, 3), ("small96", 15, 3000, True, 1100, 2)])
+def test_prefill_attention_splits(hip, oracle_threads, model, t, pos0, kv_fp16, window, splits):  # noqa: F811
+    """t queries behind pos0 filled keys: the keys over `splits` workgroups as
+    well, with ragged last steps, splits without keys for some wavefronts, up to
+    three query blocks, and windows whose first key lies far from 0.  Last
+    logits and, in the second layer (its rows follow from the first's
+    attention), K and V of the new positions."""
+    spec = SMALL96 if model == "small96" else dict(synth.SPECS[model], layers=2)
+    name = "phi3mini" if model == "small96" else model
+    assert host_fn("prefill_attn_splits", "iiiii")(t, pos0, spec["heads"], int(kv_fp16), window) == splits
+    ctx = (pos0 + t + 64) // 64 * 64
+    img = synth.build_image(name, seed=1234, spec=spec, context=ctx, sliding_window=window)
+    prompt = synth.prompt(spec["vocab"], t, seed=7)
+    pair = OraclePair(img, kv_fp16, ctx)
+    eng = InferenceEngine(LoadedModel.load(img), hip, kv_fp16=kv_fp16, context=ctx)
+    try:
+        pair.kv_fill_random(pos0, 3)
+        eng.kv_fill_random(pos0, 3)
+        want = pair.prefill(prompt, pos0)
+        got, _ = eng.prefill(prompt, pos0)
+        err = float(np.max(np.abs(got - want)))
+        worst = floor = 0.0
+        for p in range(pos0, pos0 + t):
+            rows = list(zip(eng.kv_read(1, p), pair.kv_read(1, p), *pair.kv_alt_reads(1, p)))
+            worst = max([worst] + [float(np.max(np.abs(g - r)) / np.max(np.abs(r))) for g, r, *_ in rows])
+            floor = max([floor] + [float(np.max(np.abs(o - r)) / np.max(np.abs(r))) for _, r, *alt in rows for o in alt])
+        print(f"splits {splits}: max |dlogit| {err:.3e}, KV {worst:.1e} (floor {floor:.1e})")
+        assert err <= pair.bounds()[0][0]
+        assert worst <= max(KV_MIN, KV_MARGIN * floor)
+    finally:
+        pair.close()
+        eng.dispose()
