@@ -255,3 +255,35 @@ def test_top_p_stages(hip, n, top_p, scale):
     o = opts(0.8, 0, top_p, 1.2, 64)
     for r in R_FEW:
         assert hip.sample(x, o, recent, r) == ref(x, o, recent, r), r
+
+
+@pytest.mark.parametrize("low", [-np.inf, np.finfo(np.float32).min])
+@pytest.mark.parametrize("n,k,top_p,finite", [(32000, 40, 0.95, 12), (32000, 40, 1.0, 41), (131073, 128, 1.0, 100),
+                                              (32000, 300, 1.0, 100), (9000, 0, 0.9, 20), (4096, 0, 0.95, 3),
+                                              (5000, 0, 0.9, 1), (9000, 0, 0.8, 8500)])
+def test_masked_logits(hip, low, n, k, top_p, finite):
+    """A masked vocabulary: all but `finite` logits at -inf or at float's lowest
+    value (whose scaled value overflows to -inf), fewer open tokens than k, a
+    mass histogram with one or a few occupied bins, a penalty on masked and open
+    tokens.  Exact; draws below the sum's rounding, where a token of
+    probability 0 cannot be reached."""
+    rng = np.random.default_rng(n + k + finite)
+    x = np.full(n, low, np.float32)
+    open_ = rng.choice(n, size=finite, replace=False)
+    x[open_] = rng.normal(0, 2, finite).astype(np.float32)
+    recent = [int(i) for i in open_[:3]] + [int(i) for i in rng.integers(0, n, 20)]
+    for o in (opts(0.8, k, top_p), opts(0.8, k, top_p, 1.3, 64)):
+        for r in (0.0, 0.29, 0.77, 0.99):
+            t = hip.sample(x, o, recent, r)
+            assert t == ref(x, o, recent, r), (o, r)
+            assert x[t] > low
+
+
+@pytest.mark.parametrize("n,k", [(32000, 40), (131073, 128), (32000, 129)])
+def test_top_k_infinite_logit(hip, n, k):
+    """One logit at +inf: inf - inf makes every probability NaN, no draw closes,
+    and the last of the k selected is returned, as in the reference."""
+    x = logits_for(n, n + k)
+    x[n // 3] = np.inf
+    for r in R_FEW:
+        assert hip.sample(x, opts(0.8, k), [], r) == ref(x, opts(0.8, k), [], r)
