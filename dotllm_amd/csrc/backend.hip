@@ -1164,7 +1164,7 @@ bool prefill_check(const llmdot_hip_model* m) {
     const auto& d = m->d;
     const int qdim = d.heads * d.head_dim;
     for (const auto& w : m->L) {
-        // the window is on the fp16 (MFMA) attention only: with an fp32 KV
+        // the window is in the fp16-cache attention only: with an fp32 KV
         // cache a windowed model's prompt runs through the decode step
         if (d.sliding_window > 0 && !d.kv_fp16) return false;
         const Weight* in_h[5] = {w.q, w.k, w.v, w.gate, w.up};

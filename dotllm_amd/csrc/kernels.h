@@ -102,7 +102,7 @@ hipError_t launch_stream_probe(void* buf, size_t nbytes, int mode, uint32_t* sin
 // Position bookkeeping for a captured decode step.
 hipError_t launch_set_scalar(int32_t* dst, int32_t v, hipStream_t s);
 hipError_t launch_set_scalars(int32_t* dst, int32_t v0, int32_t v1, hipStream_t s);   // dst[0], dst[1]
-// nbytes (> 0) between device memory and pinned host memory.
+// nbytes (> 0) between device memory and pinned host memory, both 16-byte aligned.
 hipError_t launch_copy_bytes(void* dst, const void* src, size_t nbytes, hipStream_t s);
 // Pinned dst (16-byte aligned): ints[0..4], then, with logits, the n logits from byte 32 on.
 hipError_t launch_publish_step(void* dst, const int32_t* ints, const float* logits, int n, hipStream_t s);
@@ -236,7 +236,7 @@ struct PfAttnArgs {
     int q_split, k_split, v_split;
     int64_t q_part, k_part, v_part;
     // per-head Q/K RmsNorm weights [head_dim] applied before RoPE (null: none)
-    // with eps; SlidingWindow (0: every earlier position)
+    // with eps; SlidingWindow (0: every earlier position; fp16 KV only)
     const float *q_norm, *k_norm;
     float eps;
     int window;

@@ -276,14 +276,10 @@ __global__ void set_scalars_kernel(int32_t* dst, int32_t v0, int32_t v1) {
     dst[1] = v1;
 }
 
-// nbytes from src to dst, one of them pinned host memory: bound by the host
-// link, so one 16-byte access per thread, all in flight at once.
-__global__ __launch_bounds__(256) void copy_bytes_kernel(uint8_t* dst, const uint8_t* src, int64_t nbytes, int wide) {
+// nbytes from src to dst (16-byte aligned), one of them pinned host memory:
+// bound by the host link, so one 16-byte access per thread, all in flight at once.
+__global__ __launch_bounds__(256) void copy_bytes_kernel(uint8_t* dst, const uint8_t* src, int64_t nbytes) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (!wide) {
-        if (i < nbytes) dst[i] = src[i];
-        return;
-    }
     if (16 * i + 16 <= nbytes) {
         reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
     } else {
@@ -441,10 +437,10 @@ hipError_t launch_set_scalars(int32_t* dst, int32_t v0, int32_t v1, hipStream_t 
     return hipGetLastError();
 }
 hipError_t launch_copy_bytes(void* dst, const void* src, size_t nbytes, hipStream_t s) {
-    const bool wide = ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) & 15) == 0;
-    const size_t items = wide ? (nbytes + 15) / 16 : nbytes;
+    if (nbytes == 0 || ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) & 15)) return hipErrorInvalidValue;
+    const size_t items = (nbytes + 15) / 16;
     copy_bytes_kernel<<<(unsigned)((items + 255) / 256), 256, 0, s>>>((uint8_t*)dst, (const uint8_t*)src,
-                                                                      (int64_t)nbytes, wide);
+                                                                      (int64_t)nbytes);
     return hipGetLastError();
 }
 hipError_t launch_publish_step(void* dst, const int32_t* ints, const float* logits, int n, hipStream_t s) {

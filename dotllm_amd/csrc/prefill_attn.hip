@@ -203,8 +203,9 @@ __global__ __launch_bounds__(64 * W) void pf_attn_wave_kernel(PfAttnArgs a) {
     at.load_q(a, tqc, h, lk);
     const int last = tq < a.T ? a.pos0 + tq : -1;   // the query's last key
     // SlidingWindow (IE:385-387): the query's first key, and the block's first step
-    const int first = a.window > 0 ? max(0, a.pos0 + tqc + 1 - a.window) : 0;
-    const int jstart = a.window > 0 ? max(0, a.pos0 + t0 + 1 - a.window) / KSTEP * KSTEP : 0;
+    const int window = F16 ? a.window : 0;   // fp16 caches only (launch_prefill_attn_wave)
+    const int first = window > 0 ? max(0, a.pos0 + tqc + 1 - window) : 0;
+    const int jstart = window > 0 ? max(0, a.pos0 + t0 + 1 - window) / KSTEP * KSTEP : 0;
     // the window's first 8 floor(len/8) keys are the Softmax's vector lanes
     const int n8 = first + ((a.pos0 + tqc + 1 - first) & ~7);
     const int nkeys = a.pos0 + min(t0 + QB, a.T);
@@ -400,6 +401,7 @@ int prefill_attn_splits(int T, int pos0, int heads, int kv_fp16, int window) {
 hipError_t launch_prefill_attn_wave(const PfAttnArgs& a, hipStream_t s) {
     if (a.splits > 1 && (!a.part_max || !a.part_out || !a.part_z || a.part_stride < (int64_t)a.T * a.heads * a.head_dim))
         return hipErrorInvalidValue;
+    if (!a.kv_fp16 && a.window > 0) return hipErrorInvalidValue;
     switch (a.head_dim) {
     case 64: return a.kv_fp16 ? launch_wave<64, true>(a, s) : launch_wave<64, false>(a, s);
     case 96: return a.kv_fp16 ? launch_wave<96, true>(a, s) : launch_wave<96, false>(a, s);
