@@ -1378,6 +1378,14 @@ namespace {
 // 4096: 128-token tiles 107, 64-token 83, in 2 parts 57; 512 x 2048 x 8192:
 // 199, in 8 parts 49; 256 x 28672 x 4096 (448 tiles): 154 in any split; Q6_K
 // 777 x 3072 x 8192 (168 tiles): 238, in 3 parts 128, 64-token tiles 222, 167.
+// The estimate is of the launch alone, and of one rate for all formats: Q6_K
+// takes three MFMAs a product, and V runs beside Q + K, so those take longer in
+// place than alone (V of 512 tokens, 1B shape, 23 against an estimated 12; Q + K
+// of 777, Phi-3-mini shape, 139 against 96).  V's choice stands beside Q + K all
+// the same, us of whole calls: 2 layers of the 7B shape, 2048 tokens, in its 4
+// parts 4991, unsplit 5047, in 2 parts 4987; 1024 tokens in 4 parts of 64-token
+// tiles 2568, unsplit 128-token tiles 2607; 4 layers of the 1B shape, 512 tokens,
+// in 8 parts 1162, unsplit 1263, in 4 parts 1150.
 double gemm_us(int tm, int M, int N, int steps, double parts, int sp) {
     const double alone = tm == 32 ? 0.47 : tm == 64 ? 0.58 : 0.80;
     const double two = tm == 32 ? 0.58 : tm == 64 ? 0.77 : 1.15;
